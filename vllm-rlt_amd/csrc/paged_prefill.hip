@@ -153,12 +153,23 @@ __device__ __forceinline__ void seq_rows(const PrefillArgs& a, int s, int& row0,
 // first.  Workgroup b runs on XCD b % 8 (the dispatcher's round-robin) and is
 // that XCD's (b / 8)-th item; each XCD's queue walks the ranked sequences, for
 // each its heads h == xcd (mod 8), and for each head the query tiles, last
-// (longest) first.  So the dispatcher hands out the longest items first on
+// (longest) first.  Ranking costs one memory round trip plus a step per
+// sequence: up to kWaveSeqs of them every wave ranks alone in registers (0.8
+// us of an item at 8 sequences; a readlane step is ~45 ns, so 64 of them took
+// 3.0 us against 1.2 us through LDS), beyond that the threads share the costs
+// through LDS (1.8 us at 128 sequences, 5.1 us with a sort and a scan behind
+// barriers).  So the dispatcher hands out the longest items first on
 // every XCD (greedy LPT), and the query tiles that stream one (sequence,
 // head)'s prefix run back to back on one XCD, sharing its L2.  Direct mode:
 // item = (seq * max_qt + t) * hq + head; empty items exit.
 constexpr int kXcds = 8;
-constexpr int kRankSeqs = 512;  // ranked mode: at most this many sequences
+constexpr int kRankSeqs = 512;  // ranked mode: at most this many sequences (one per thread)
+constexpr int kWaveSeqs = 16;   // ranked by every wave in registers up to here, through LDS above
+
+// Key tiles of a sequence of len keys: what its longest query tile costs.
+__device__ __forceinline__ uint32_t rank_cost(int len) {
+  return len > 0 ? (static_cast<uint32_t>(len) + kBN - 1) / kBN : 0u;
+}
 constexpr int kTablePages = 4096;  // page ids staged in LDS per workgroup (65536 keys)
 
 template <typename T, int D, bool DMA>
@@ -184,11 +195,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   constexpr int PAGES_PER_PASS = TOKENS_PER_PASS / kPage;
   constexpr int PASSES = kBN / TOKENS_PER_PASS;
   constexpr int TILES_PER_CHUNK = 64 / (kBN / kPage);  // table entries arrive 64 at a time
-  constexpr int MERGE_FLOATS = 2 + 16 * DTILES;        // m, l, accumulators per lane
   static_assert(kBN % TOKENS_PER_PASS == 0 && TOKENS_PER_PASS % kPage == 0, "tile loads");
   static_assert(64 % CHUNKS == 0 && (64 / CHUNKS) <= kPage, "a wave's loads stay in one page");
-  static_assert(4 * 64 * MERGE_FLOATS * 4 <= 4 * (KT + VT) * 2, "merge fits in the tile buffers");
-  static_assert(4 * kRankSeqs * 4 <= 4 * (KT + VT) * 2, "ranking fits in the tile buffers");
+  static_assert((2 * kRankSeqs + 2) * 4 <= 4 * (KT + VT) * 2, "ranking fits in the tile buffers");
   // Two key groups, each with two K and V tile buffers; reused for ranking
   // before the tile loop and for the key-group merge after it.
   __shared__ __align__(16) uint16_t lds[4 * (KT + VT)];
@@ -197,69 +206,107 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   __shared__ int32_t page_ids[DMA ? kTablePages : 1];
 
   const int tid = threadIdx.x;
-  int seq, t, h;
+  const int lane = tid & 63;
+  const int wave = uniform(tid >> 6);  // scalar, so per-wave conditions branch on SCC
+  const int64_t max_len = a.width * kPage;
+  int seq, t, h, row0, nq, len_k;
   if (a.ranked) {
-    int* s_qt = reinterpret_cast<int*>(lds);  // [kRankSeqs] query tiles per sequence
-    int* s_cost = s_qt + kRankSeqs;            // key tiles of its last query tile
-    int* s_order = s_cost + kRankSeqs;         // sequences, longest first
-    int* s_scan = s_order + kRankSeqs;         // query tiles of the ranked sequences, prefix sums
-    const int ns = a.num_seqs;
-    if (tid < ns) {
-      int r0, nq_s;
-      seq_rows(a, tid, r0, nq_s);
-      const int keys = static_cast<int>(min<int64_t>(a.lens[tid], a.width * kPage));
-      s_qt[tid] = (nq_s + kBM - 1) / kBM;
-      s_cost[tid] = keys > 0 ? (keys + kBN - 1) / kBN : 0;
-    }
-    __syncthreads();
-    if (tid < ns) {
-      const int c = s_cost[tid];
-      int r = 0;
-      for (int q = 0; q < ns; ++q) {
-        const int cq = s_cost[q];
-        r += (cq > c) || (cq == c && q < tid);
-      }
-      s_order[r] = tid;
-    }
-    __syncthreads();
-    s_scan[tid] = tid < ns ? s_qt[s_order[tid]] : 0;
-    __syncthreads();
-    for (int off = 1; off < ns; off <<= 1) {  // inclusive scan of the ns ranked entries
-      const int v = tid >= off ? s_scan[tid - off] : 0;
-      __syncthreads();
-      s_scan[tid] += v;
-      __syncthreads();
-    }
     // XCD b % 8 owns heads h == b % 8 (mod 8): hpx of them per sequence.
+    // Sequence s covers positions [hpx * before, hpx * (before + qt)) of every
+    // XCD's queue, `before` being the query tiles of the sequences ranked
+    // ahead of it.
+    const int ns = a.num_seqs;
     const int hpx = a.hq / kXcds;
     const int xcd = static_cast<int>(blockIdx.x) % kXcds;
     const int pos = static_cast<int>(blockIdx.x) / kXcds;
-    // Ranked sequence r covers positions [hpx * scan[r-1], hpx * scan[r]).
-    int lo = 0, hi = ns;  // first r with hpx * scan[r] > pos
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (hpx * s_scan[mid] > pos) hi = mid;
-      else lo = mid + 1;
+    int before = 0, qt;
+    if (ns <= kWaveSeqs) {
+      // One sequence per lane, every wave on its own: a memory round trip and
+      // kWaveSeqs steps in registers, no barrier.
+      const int s = min(lane, ns - 1);
+      int r0, n;
+      seq_rows(a, s, r0, n);
+      const int len = static_cast<int>(min<int64_t>(a.lens[s], max_len));
+      const int tiles = (n + kBM - 1) / kBM;
+      const uint32_t key = rank_cost(len) * kWaveSeqs + (kWaveSeqs - 1 - s);
+      // Lanes past ns hold copies of the last sequence: q >= ns counts nothing.
+      const int mine = lane < ns ? tiles : 0;
+#pragma unroll
+      for (int q = 0; q < kWaveSeqs; ++q) {
+        const uint32_t kq = __builtin_amdgcn_readlane(key, q);
+        before += kq > key ? __builtin_amdgcn_readlane(mine, q) : 0;
+      }
+      const uint64_t hit =
+          __builtin_amdgcn_ballot_w64(lane < ns && pos >= hpx * before && pos < hpx * (before + tiles));
+      if (hit == 0) return;
+      seq = __builtin_ctzll(hit);
+      before = __builtin_amdgcn_readlane(before, seq);
+      qt = __builtin_amdgcn_readlane(tiles, seq);
+      row0 = __builtin_amdgcn_readlane(r0, seq);
+      nq = __builtin_amdgcn_readlane(n, seq);
+      len_k = __builtin_amdgcn_readlane(len, seq);
+    } else {
+      // One sequence per thread, costs and tiles exchanged through LDS.
+      uint32_t* s_key = reinterpret_cast<uint32_t*>(lds);        // [kRankSeqs] cost, then index
+      int* s_qt = reinterpret_cast<int*>(s_key + kRankSeqs);     // [kRankSeqs] query tiles
+      int* s_hit = s_qt + kRankSeqs;                             // the workgroup's sequence: index, before
+      int tiles = 0;
+      uint32_t key = 0;
+      if (tid < ns) {
+        int r0, n;
+        seq_rows(a, tid, r0, n);
+        tiles = (n + kBM - 1) / kBM;
+        // 23 bits of cost: longer contexts (over 2^29 keys) rank by index.
+        const uint32_t cost = rank_cost(static_cast<int>(min<int64_t>(a.lens[tid], max_len)));
+        key = min(cost, (1u << 23) - 1) * kRankSeqs + (kRankSeqs - 1 - tid);
+      }
+      s_key[tid] = key;  // slots past ns count nothing
+      s_qt[tid] = tiles;
+      if (tid == 0) s_hit[0] = -1;
+      __syncthreads();
+      if (tid < ns) {
+        for (int q = 0; q < ns; q += 16) {
+          u32x4 k4[4], w4[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            k4[i] = *reinterpret_cast<const u32x4*>(s_key + q + 4 * i);
+            w4[i] = *reinterpret_cast<const u32x4*>(s_qt + q + 4 * i);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) before += k4[i][e] > key ? static_cast<int>(w4[i][e]) : 0;
+        }
+        if (pos >= hpx * before && pos < hpx * (before + tiles)) {
+          s_hit[0] = tid;
+          s_hit[1] = before;
+        }
+      }
+      __syncthreads();
+      seq = uniform(s_hit[0]);
+      if (seq < 0) return;
+      before = uniform(s_hit[1]);
+      qt = uniform(s_qt[seq]);
+      seq_rows(a, seq, row0, nq);
+      len_k = static_cast<int>(min<int64_t>(a.lens[seq], max_len));
+      __syncthreads();  // the ranking arrays are dead before the tiles reuse them
     }
-    if (lo >= ns) return;
-    seq = s_order[lo];
-    const int qt = s_qt[seq];
-    const int local = pos - hpx * (lo > 0 ? s_scan[lo - 1] : 0);
+    const int local = pos - hpx * before;
     h = xcd + kXcds * (local / qt);
     t = qt - 1 - local % qt;
-    __syncthreads();  // ranking arrays are dead before the tiles reuse them
   } else {
     const int w = blockIdx.x;
     h = w % a.hq;
     seq = w / a.hq / a.max_qt;
     t = w / a.hq % a.max_qt;
     if (seq >= a.num_seqs) return;
+    seq_rows(a, seq, row0, nq);
+    if (t * kBM >= nq) return;
+    len_k = static_cast<int>(min<int64_t>(a.lens[seq], max_len));
   }
-  int row0, nq;
-  seq_rows(a, seq, row0, nq);
-  if (t * kBM >= nq) return;
-  const int64_t max_len = a.width * kPage;
-  const int len_k = static_cast<int>(min<int64_t>(a.lens[seq], max_len));
+  // Scalar from here on: the tile loop branches on them.
+  seq = uniform(seq), t = uniform(t), h = uniform(h);
+  row0 = uniform(row0), nq = uniform(nq), len_k = uniform(len_k);
   const int prefix = len_k - nq;
   const int kvh = h / (a.hq / a.hkv);
   const int qt0 = t * kBM;                         // first chunk row of the workgroup
@@ -280,8 +327,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
 
   // Waves 0-3 take key tiles 0, 2, 4, ...; waves 4-7 tiles 1, 3, 5, ...; wave
   // w and w + 4 own the same 32 query rows and merge at the end.
-  const int lane = tid & 63;
-  const int wave = uniform(tid >> 6);  // scalar, so per-wave conditions branch on SCC
   const int kg = wave >> 2;   // key group
   const int qw = wave & 3;    // query wave within the group
   const int gtid = tid & 255; // thread within the key group
@@ -297,12 +342,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
 
   // Q^T B-operands: lane holds dims [ks*16 + half*8, +8) of query my_row.
   u32x4 qb[KSTEPS];
-  {
+  auto load_q = [&]() __attribute__((always_inline)) {
     const int r = row0 + min(my_row, nq - 1);
     const T* qrow = static_cast<const T*>(a.q) + r * a.q_row + static_cast<int64_t>(h) * a.q_head;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) qb[ks] = *reinterpret_cast<const u32x4*>(qrow + ks * 16 + half * 8) ^ a.q_sign;
-  }
+  };
 
   // Tile loads: pass i of tile j reads page 4j + i*PAGES_PER_PASS + ld_page,
   // the same page for the whole wave, so its table entry and base address are
@@ -336,11 +381,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
     return static_cast<uint32_t>((min(slot, slot_limit) * a.kv_token + chunk * 8) * sizeof(T));
   };
   // Page p of the sequence (p < 4 * ntiles, which the host keeps within
-  // kTablePages); past the last valid page the last page's id.  page_slot
-  // reads the entry into a vector register (its use can come a phase later),
-  // page_id makes it scalar.
+  // kTablePages) from the LDS copy; past the last valid page the last page's
+  // id.  The value stays in a vector register: its use can come a phase later.
   auto page_slot = [&](int p) -> int32_t { return page_ids[min(p, kTablePages - 1)]; };
-  auto page_id = [&](int p) -> uint32_t { return static_cast<uint32_t>(uniform(page_slot(p))); };
   // Page p of tile j that wave qw stages; tiles past the last are clamped.
   auto tile_page = [&](int j) { return min(j, ntiles - 1) * (kBN / kPage) + qw; };
   // Per-lane source offsets of the four staging instructions of a page, and
@@ -602,16 +645,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int niter = (ntiles + 1) / 2;  // tiles per key group (the last of group 1 may not exist)
 
   if constexpr (DMA) {
-    const int fill = min(4 * ntiles, kTablePages);
-    for (int i = tid; i < fill; i += 512) page_ids[i] = trow[min(i, last_page)];
-    {
-      // The V tile of buffer 1, which the first MFMA phase reads (times P = 0)
-      // before any tile is staged there: zero, so no stale NaN reaches acc_o.
-      u32x4* vz = reinterpret_cast<u32x4*>(group_lds + (KT + VT) + KT);
-      const u32x4 zero = {0u, 0u, 0u, 0u};
-      for (int i = tid & 255; i < VT / 8; i += 256) vz[i] = zero;
-    }
-    __syncthreads();
     // Ping-pong.  Iteration t of key group g handles tile j = 2t + g in two
     // phases: an MFMA phase (P V of tile j - 2, then S of tile j) and a
     // softmax phase (tile j's exponentials, with the staging DMA of K of tile
@@ -626,8 +659,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
     // last tile they re-read it into buffers no later phase reads), so at the
     // barrier before MFMA phase t, vmcnt(8) completes everything issued
     // before the previous softmax phase -- the K of tile j and V of tile j - 2
-    // that this phase reads (loads return in order).  The prologue issues
-    // K(j), V(j), K(j + 2): vmcnt(8) there completes K(j).  Page ids run down
+    // that this phase reads (loads return in order).  The prologue waits for
+    // K(j), then issues V(j) and K(j + 2): vmcnt(8) passes them at t = 0.  Page ids run down
     // a chain (V <- K <- next), so each phase reads one new id from LDS, a
     // phase before its use.  No load here is a bare L2 prefetch of a later
     // tile: with in-order completion, the barrier's vmcnt would wait for its
@@ -642,13 +675,57 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
     };
-    issue_half(tile_page(kg), page_id(tile_page(kg)), 0, 0);
-    issue_half(tile_page(kg), page_id(tile_page(kg)), 0, 1);
-    issue_half(tile_page(kg + 2), page_id(tile_page(kg + 2)), 1, 0);
+    // Prologue.  One memory round trip fetches q (whole rows, straight into
+    // the V halves of the two groups' buffers 1, swizzled like K rows), the
+    // page ids of the wave's first four tiles (scalar loads) and the copy of
+    // all page ids for LDS; a second one the first K tile.  V of that tile and
+    // K of the next go out before the first MFMA phase and land under it.
+    // What an item spends outside its tile loop is latency: one of two key
+    // tiles (chunk 128, no prefix) takes 10.2 us, against 15.1 us when q came
+    // as 32-byte pieces of rows, the ids behind a barrier of their own and
+    // three tiles were awaited; 64 such sequences 77.7 -> 49.6 us a launch.
+    const auto* srow = reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(trow));
+    uint32_t first_id[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) first_id[i] = static_cast<uint32_t>(srow[min(tile_page(kg + 2 * i), last_page)]);
+    const int fill = min(4 * ntiles, kTablePages);
+    constexpr int kCopy = 3;  // page ids in flight per thread beside the first tile
+    int32_t ids[kCopy];
+#pragma unroll
+    for (int u = 0; u < kCopy; ++u) ids[u] = trow[min(u * 512 + tid, last_page)];
     __builtin_amdgcn_sched_barrier(0);
-    uint32_t id_v = page_id(tile_page(kg + 2));        // V of tile j + 2
-    uint32_t id_k = page_id(tile_page(kg + 4));        // K of tile j + 4
-    int32_t next_k = page_slot(tile_page(kg + 6));     // K of tile j + 6
+    {
+      const uint64_t qbase = static_cast<uint64_t>(uniform64(reinterpret_cast<int64_t>(
+          static_cast<const T*>(a.q) + (row0 + qt0) * a.q_row + static_cast<int64_t>(h) * a.q_head)));
+      const uint32_t dst = lds_address(group_lds + (KT + VT) + KT + qw * 16 * KROW);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * wave + 4 * i + (lane >> 4);
+        const int chunk = (lane & 15) ^ lds_swizzle(4 * i + (lane >> 4));
+        lds_dma16(dst + i * 4 * KROW * sizeof(uint16_t),
+                  static_cast<uint32_t>((min(r, nq - 1 - qt0) * a.q_row + chunk * 8) * sizeof(T)), qbase);
+      }
+    }
+    issue_half(tile_page(kg), first_id[0], 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kCopy; ++u)
+      if (u * 512 + tid < fill) page_ids[u * 512 + tid] = ids[u];
+    for (int i = kCopy * 512 + tid; i < fill; i += 512) page_ids[i] = trow[min(i, last_page)];
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    {
+      const char* rows =
+          reinterpret_cast<const char*>(lds + (2 * (qw >> 1) + 1) * (KT + VT) + KT + 32 * (qw & 1) * KROW);
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+        qb[ks] = *reinterpret_cast<const u32x4*>(rows + (((ks << 5) ^ k_key) + k_base)) ^ a.q_sign;
+    }
+    issue_half(tile_page(kg), first_id[0], 0, 1);
+    issue_half(tile_page(kg + 2), first_id[1], 1, 0);
+    uint32_t id_v = first_id[1];                             // V of tile j + 2
+    uint32_t id_k = first_id[2];                             // K of tile j + 4
+    int32_t next_k = static_cast<int32_t>(first_id[3]);      // K of tile j + 6
+    __builtin_amdgcn_sched_barrier(0);
     if (kg == 1) phase_barrier();
     f32x16 sacc[2] = {{}, {}};  // P of tile j - 2: none before the first phase
     bool rescale = false;
@@ -659,12 +736,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
       load_barrier();
       __builtin_amdgcn_s_setprio(1);
       // One site for the whole phase (accumulators updated on two paths would
-      // be given two register sets).  At t = 0 the P V half multiplies a
-      // zeroed V buffer by P = 0; past the wave's last tile, and at t = niter,
-      // the S half's scores are never used.
+      // be given two register sets).  At t = 0 the P V half multiplies what
+      // buffer 1 holds by P = 0 and its accumulators are cleared afterwards (a
+      // NaN times 0); past the wave's last tile, and at t = niter, the S
+      // half's scores are never used.
       if (t == 0 ? active(j) : active(j - 2))
         mfma_phase(std::true_type{}, std::true_type{}, 1 - P, P, sacc, rescale, corr);
       __builtin_amdgcn_s_setprio(0);
+      if (t == 0) {
+#pragma unroll
+        for (int c = 0; c < DTILES; ++c) acc_o[c] = f32x16{};
+      }
       if (t == niter) break;
       phase_barrier();
       const uint32_t id_next = static_cast<uint32_t>(uniform(next_k));
@@ -706,6 +788,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
         *reinterpret_cast<u32x4*>(&vb[tok * VROW + ld_chunk * 8]) = vreg[i];
       }
     };
+    load_q();
     if (kg < ntiles) {
       load_tile(kg);
       store_tile(0);
@@ -727,45 +810,76 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
     }
   }
 
-  // Merge the key groups: group 1 hands (m, l, acc) to group 0 through LDS,
-  // laid out [query wave][value][lane] (the last barrier ordered every tile
-  // read before these writes).
-  float* xs = reinterpret_cast<float*>(lds) + qw * MERGE_FLOATS * 64 + lane;
-  if (kg == 1) {
-    xs[0] = m;
-    xs[64] = lsum;
+  // Merge the key groups (2.7 us an item with the stores; 3.7 us when group 0
+  // merged alone and stored 8 bytes of 32 rows per instruction).  Each keeps
+  // half of the output columns: group 0 the
+  // first DTILES / 2 tiles of 32 dims, group 1 the rest, and hands the other
+  // group its (m, l) and the accumulators of the half it does not keep (the
+  // last barrier ordered every tile read before these writes).
+  constexpr int HT = DTILES / 2;
+  constexpr int XCHG = 2 + 16 * HT;  // floats per lane handed over
+  static_assert(DTILES % 2 == 0, "each key group merges half of the columns");
+  f32x4* const xacc = reinterpret_cast<f32x4*>(lds);                          // [8 waves][4 HT][64]
+  float2* const xml = reinterpret_cast<float2*>(xacc + 8 * 4 * HT * 64);      // [8 waves][64]
+  uint16_t* const xrow = reinterpret_cast<uint16_t*>(xml + 8 * 64);           // [8 waves][32][OROW]
+  constexpr int OROW = 32 * HT + 8;  // padded output rows of a wave's half, elements
+  static_assert(8 * 64 * XCHG * 4 + 8 * 32 * OROW * 2 <= 4 * (KT + VT) * 2, "merge fits in the tile buffers");
+  f32x16 keep[HT];
 #pragma unroll
-    for (int c = 0; c < DTILES; ++c)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) xs[(2 + c * 16 + r) * 64] = acc_o[c][r];
-  }
-  __syncthreads();
-  if (kg == 1) return;
-  float total;  // the row's sum of P
-  {
-    const float m1 = xs[0];
-    const float mm = fmaxf(m, m1);
-    const float c0 = (m == -INFINITY) ? 0.f : fast_exp2(m - mm);
-    const float c1 = (m1 == -INFINITY) ? 0.f : fast_exp2(m1 - mm);
-    total = lsum * c0 + xs[64] * c1;
-    total += __shfl_xor(total, 32, 64);  // the two halves hold the row's two key halves
-#pragma unroll
-    for (int c = 0; c < DTILES; ++c)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc_o[c][r] = acc_o[c][r] * c0 + xs[(2 + c * 16 + r) * 64] * c1;
-  }
-
-  if (!wave_live || !row_valid) return;
-  const float inv = total > 0.f ? 1.f / total : 0.f;  // a row that sees no key is written as zeros
-  T* orow = static_cast<T*>(a.out) + (row0 + my_row) * a.o_row + static_cast<int64_t>(h) * a.o_head;
-#pragma unroll
-  for (int c = 0; c < DTILES; ++c)
+  for (int c = 0; c < HT; ++c) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const u32x2 w2 = {Ops::pack2(acc_o[c][g * 4] * inv, acc_o[c][g * 4 + 1] * inv),
-                        Ops::pack2(acc_o[c][g * 4 + 2] * inv, acc_o[c][g * 4 + 3] * inv)};
-      *reinterpret_cast<u32x2*>(orow + c * 32 + g * 8 + half * 4) = w2;
+      f32x4 give;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = acc_o[c][4 * g + e], hi = acc_o[HT + c][4 * g + e];
+        give[e] = kg == 0 ? hi : lo;
+        keep[c][4 * g + e] = kg == 0 ? lo : hi;
+      }
+      xacc[((wave * HT + c) * 4 + g) * 64 + lane] = give;
     }
+  }
+  xml[wave * 64 + lane] = make_float2(m, lsum);
+  __syncthreads();
+  float total;  // the row's sum of P
+  {
+    const float2 other = xml[(wave ^ 4) * 64 + lane];
+    const float mm = fmaxf(m, other.x);
+    const float c0 = (m == -INFINITY) ? 0.f : fast_exp2(m - mm);
+    const float c1 = (other.x == -INFINITY) ? 0.f : fast_exp2(other.x - mm);
+    total = lsum * c0 + other.y * c1;
+    total += __shfl_xor(total, 32, 64);  // the two halves hold the row's two key halves
+#pragma unroll
+    for (int c = 0; c < HT; ++c)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = xacc[(((wave ^ 4) * HT + c) * 4 + g) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) keep[c][4 * g + e] = keep[c][4 * g + e] * c0 + x[e] * c1;
+      }
+  }
+  if (!wave_live) return;
+  // Through the wave's own LDS rows, so that a store instruction writes whole
+  // runs of a row's half (16 bytes per lane) instead of 8 bytes of 32 rows.
+  const float inv = total > 0.f ? 1.f / total : 0.f;  // a row that sees no key is written as zeros
+  uint16_t* const rows = xrow + wave * 32 * OROW;
+#pragma unroll
+  for (int c = 0; c < HT; ++c)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const u32x2 w2 = {Ops::pack2(keep[c][g * 4] * inv, keep[c][g * 4 + 1] * inv),
+                        Ops::pack2(keep[c][g * 4 + 2] * inv, keep[c][g * 4 + 3] * inv)};
+      *reinterpret_cast<u32x2*>(rows + col * OROW + c * 32 + g * 8 + half * 4) = w2;
+    }
+  constexpr int OCH = 4 * HT;        // 16-byte chunks of a row's half
+  constexpr int ORPI = 64 / OCH;     // rows per store instruction
+  T* const obase = static_cast<T*>(a.out) + (row0 + wave_row0) * a.o_row + static_cast<int64_t>(h) * a.o_head + kg * 32 * HT;
+#pragma unroll
+  for (int i = 0; i < 32 / ORPI; ++i) {
+    const int r = i * ORPI + lane / OCH;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(rows + r * OROW + (lane % OCH) * 8);
+    if (wave_row0 + r < nq) *reinterpret_cast<u32x4*>(obase + r * a.o_row + (lane % OCH) * 8) = v;
+  }
 }
 
 int64_t expand_bytes(int64_t total_q, int64_t width) {
@@ -874,7 +988,9 @@ extern "C" int rlt_paged_prefill(const void* q, const int64_t* q_strides, const 
     const dim3 grid(static_cast<unsigned>(items));
     hipStream_t st = as_stream(stream);
     // Direct-to-LDS staging needs the key range's page ids to fit in LDS.
-    const bool dma = head_dim == 128 && max_table_width <= kTablePages;
+    // (and a workgroup's query rows within 32-bit offsets).
+    const bool dma = head_dim == 128 && max_table_width <= kTablePages && q_strides[0] >= 0 &&
+                     q_strides[0] * esize * kBM < (int64_t(1) << 31);
     if (dtype == RLT_BFLOAT16) {
       if (dma) hipLaunchKernelGGL((paged_prefill_mfma_kernel<bf16, 128, true>), grid, dim3(512), 0, st, p);
       else if (head_dim == 128) hipLaunchKernelGGL((paged_prefill_mfma_kernel<bf16, 128, false>), grid, dim3(512), 0, st, p);
