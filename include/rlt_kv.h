@@ -364,6 +364,37 @@ int rlt_paged_prefill(const void* q, const int64_t* q_strides, const void* key_c
                       void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * rlt_paged_prefill with room for key segments.  Same arguments, contract and
+ * refusals.  On the MFMA path (head_dim 128), a launch of few query tiles over
+ * long contexts has the sequences' keys cut into segments that run side by
+ * side, each row's segment partials in `workspace`, merged by a second kernel.
+ * Whether and how often depends on the launch's shapes (total_q, num_seqs,
+ * max_table_width, num_q_heads) and each sequence's length, so a row's last
+ * bits may depend on how many query rows share its launch; rlt_paged_prefill,
+ * or a workspace below rlt_paged_prefill_split_workspace_bytes() (or NULL),
+ * never cuts.  The workspace must not be shared by calls that overlap.  Off
+ * the MFMA path the workspace is rlt_paged_prefill's, and its size the same.
+ */
+int rlt_paged_prefill_split(const void* q, const int64_t* q_strides, const void* key_cache,
+                            const void* value_cache, const int64_t* kv_strides,
+                            const int32_t* block_tables, int64_t table_stride,
+                            int64_t max_table_width, const int32_t* context_lengths,
+                            const int32_t* cu_seqlens_q, int64_t num_seqs, int64_t total_q,
+                            int64_t max_seqlen_q, void* out, const int64_t* out_strides,
+                            int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
+                            int64_t page_size, int64_t num_blocks, float scale, int dtype,
+                            void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
+ * Workspace bytes rlt_paged_prefill_split needs to cut key ranges (shape-only;
+ * 0 when no sequence of these shapes is cut, at most 17 MB otherwise).
+ */
+int64_t rlt_paged_prefill_split_workspace_bytes(int64_t total_q, int64_t num_seqs,
+                                                int64_t max_table_width, int64_t num_q_heads,
+                                                int64_t num_kv_heads, int64_t head_dim,
+                                                int64_t page_size, int dtype);
+
+/*
  * Batched LAST-EXITED exit copies from device-resident descriptors.
  * Replaces finalize_kernel, vllm_rlt/kernels/routing.py:80-109 (launched at
  * vllm_rlt/worker/model_runner.py:543-557).  For every descriptor i with

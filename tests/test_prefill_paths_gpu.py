@@ -72,3 +72,56 @@ def test_query_rows_far_apart():
     run_prefill(wide, kp, vp, tables, lens, cu, chunks, out=out)
     atol, rtol = TOL[torch.bfloat16]
     torch.testing.assert_close(out.cpu(), paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "hq,hkv,prefixes,chunks",
+    [
+        (8, 8, [2047], [1]),  # one row, every segment full
+        (8, 2, [959, 1022, 1025], [1, 2, 3]),  # 15, 16 and 17 key tiles: two segments from 16 on
+        (16, 16, [3000], [130]),  # two query tiles; the last segment is cut short
+        (16, 4, [5000, 0, 40], [64, 33, 7]),  # a long sequence beside ones too short to cut
+        (8, 8, [0], [1500]),  # no prefix: the first query tiles end before the later segments
+        (32, 8, [2600, 130], [129, 128]),
+    ],
+)
+def test_cut_key_ranges(dtype, hq, hkv, prefixes, chunks):
+    # Few query tiles over long contexts: keys in segments and a merge.  The
+    # workspace starts as NaN, so a partial that is read is one that was written.
+    from vllm_rlt_amd import ops
+
+    q, kp, vp, tables, lens, cu, row_tables, row_lengths = ragged_prefill_case(dtype, hq, hkv, 128, prefixes, chunks, 21)
+    need = ops.prefill_split_workspace_bytes(len(q), len(chunks), tables.shape[1], hq, hkv, 128, 16, dtype)
+    assert 0 < need <= 17 << 20
+    print(f"[prefill cut] {hq}/{hkv} prefixes={prefixes} chunks={chunks} {dtype}", flush=True)
+    args = [t.cuda() for t in (q, kp, vp, tables, lens, cu)]
+    workspace = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    out = ops._paged_prefill(*args, max(chunks), None, None, workspace, True)
+    plain = ops.paged_prefill(*args, max(chunks), workspace=workspace)  # a given workspace: never cut
+    torch.cuda.synchronize()
+    atol, rtol = TOL[dtype]
+    expect = paged_attention_cpu(q, kp, vp, row_tables, row_lengths)
+    torch.testing.assert_close(out.cpu(), expect, atol=atol, rtol=rtol)
+    torch.testing.assert_close(plain.cpu(), expect, atol=atol, rtol=rtol)
+    assert torch.equal(ops.paged_prefill(*args, max(chunks)), out)
+
+
+def test_cut_key_ranges_beside_a_context_shorter_than_its_chunk():
+    # Rows that see no key are zeros whether or not another sequence is cut.
+    from vllm_rlt_amd import ops
+
+    chunks, contexts = [300, 16, 5], [3, 1500, 1]
+    q, kp, vp, tables, _, cu, row_tables, _ = ragged_prefill_case(torch.bfloat16, 8, 8, 128, [0, 1484, 0], chunks, 5)
+    row_lengths = torch.tensor(
+        [max(0, n - (c - 1 - i)) for n, c in zip(contexts, chunks) for i in range(c)], dtype=torch.int32
+    )
+    out = torch.full(q.shape, 7.0, dtype=q.dtype, device="cuda")
+    ops.paged_prefill(
+        q.cuda(), kp.cuda(), vp.cuda(), tables.cuda(), torch.tensor(contexts, dtype=torch.int32).cuda(), cu.cuda(),
+        max(chunks), out=out,
+    )
+    torch.cuda.synchronize()
+    atol, rtol = TOL[torch.bfloat16]
+    torch.testing.assert_close(out.cpu(), paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
+    assert torch.count_nonzero(out.cpu()[row_lengths == 0]) == 0

@@ -138,6 +138,13 @@ struct PrefillArgs {
   int max_qt;       // direct mode: query tiles per sequence bound
   float qscale;     // |scale| * log2(e)
   uint32_t q_sign;  // 0x80008000 negates q (a negative scale), else 0
+  // Key segments (1 when no sequence is cut): per row of a cut sequence, head
+  // and segment g one partial.  With P = head * max_seg + g, the 16-byte quad j
+  // of row i's accumulator is part_acc[(P * D / 4 + j) * total_q + i] and its
+  // (max in log2 units, sum) part_ml[P * total_q + i].
+  f32x4* part_acc;
+  float2* part_ml;
+  int max_seg;  // segments of a sequence long enough for them
 };
 
 // Rows [row0, row0 + nq) of sequence s, clamped to [0, total_q] so that an
@@ -147,30 +154,166 @@ __device__ __forceinline__ void seq_rows(const PrefillArgs& a, int s, int& row0,
   nq = min(max(a.cu[s + 1], row0), a.total_q) - row0;
 }
 
-// Work list.  A work item is (sequence, query tile of kBM rows, query head).
-// Ranked mode (few sequences, hq a multiple of the XCD count): every workgroup
-// ranks the sequences by the key tiles of their last query tile, longest
-// first.  Workgroup b runs on XCD b % 8 (the dispatcher's round-robin) and is
-// that XCD's (b / 8)-th item; each XCD's queue walks the ranked sequences, for
-// each its heads h == xcd (mod 8), and for each head the query tiles, last
-// (longest) first.  Ranking costs one memory round trip plus a step per
-// sequence: up to kWaveSeqs of them every wave ranks alone in registers (0.8
-// us of an item at 8 sequences; a readlane step is ~45 ns, so 64 of them took
-// 3.0 us against 1.2 us through LDS), beyond that the threads share the costs
-// through LDS (1.8 us at 128 sequences, 5.1 us with a sort and a scan behind
-// barriers).  So the dispatcher hands out the longest items first on
-// every XCD (greedy LPT), and the query tiles that stream one (sequence,
-// head)'s prefix run back to back on one XCD, sharing its L2.  Direct mode:
-// item = (seq * max_qt + t) * hq + head; empty items exit.
+// Key segments.  A launch of few query tiles over long contexts is few work
+// items, each a long serial walk, on a chip that is mostly idle: their keys
+// are then cut into segments, every one a work item, and a merge kernel
+// combines the partials.  The host allows max_seg segments, as many as bring
+// the launch to one item per CU; a sequence takes them as long as a segment
+// keeps kSegTiles key tiles (4 iterations of two, ~6 us, against the ~10 us
+// that an item spends outside its loop).  One 512-token chunk over 16000 keys:
+// 194 -> 94 us in 4 segments; 100 tokens over 8192 keys 123 -> 31 us
+// in 16.  With 256 items already there nothing is cut: four 512-token
+// chunks over 8192 keys took 158 us uncut and 180 us in halves, the chip being
+// at its power limit either way.
+constexpr int kCus = 256;
+constexpr int kSegTiles = 8;
+constexpr int kMaxSeg = 16;
+
+// Key tiles of len keys.
+__device__ __forceinline__ int key_tiles(int len) { return len > 0 ? (len - 1) / kBN + 1 : 0; }
+
+// Segments of a sequence of len keys, 1 <= n <= max_seg.
+__device__ __forceinline__ int seq_segments(int len, int max_seg) {
+  return max(1, min(key_tiles(len) / kSegTiles, max_seg));
+}
+
+// Key tiles of one segment: an even count, so a segment's tiles alternate
+// between the key groups as the whole range's do.
+__device__ __forceinline__ int segment_tiles(int len, int n) {
+  const int tiles = key_tiles(len);
+  return n <= 1 ? tiles : ((tiles + n - 1) / n + 1) / 2 * 2;
+}
+
+// Work list.  A work item is (sequence, query tile of kBM rows, key segment,
+// query head).  Ranked mode (few sequences, hq a multiple of the XCD count):
+// every workgroup ranks the sequences by the key tiles of their longest item,
+// longest first.  Workgroup b runs on XCD b % 8 (the dispatcher's round-robin)
+// and is that XCD's (b / 8)-th item; each XCD's queue walks the ranked
+// sequences, for each its heads h == xcd (mod 8), for each head the segments
+// and for each segment the query tiles, last (longest) first.  So the
+// dispatcher hands out the longest items first on every XCD (greedy LPT), and
+// the query tiles that stream one (sequence, head)'s keys run back to back on
+// one XCD, sharing its L2.  Ranking costs one memory round trip plus a step
+// per sequence: up to kWaveSeqs of them every wave ranks alone in registers
+// (0.8 us of an item at 8 sequences; a readlane step is ~45 ns, so 64 of them
+// took 3.0 us against 1.2 us through LDS), beyond that the threads share the
+// costs through LDS (1.8 us at 128 sequences, 5.1 us with a sort and a scan
+// behind barriers).  Direct mode: item = (seq * max_qt + t) * hq + head; empty
+// items exit, and no sequence is cut.
 constexpr int kXcds = 8;
 constexpr int kRankSeqs = 512;  // ranked mode: at most this many sequences (one per thread)
 constexpr int kWaveSeqs = 16;   // ranked by every wave in registers up to here, through LDS above
-
-// Key tiles of a sequence of len keys: what its longest query tile costs.
-__device__ __forceinline__ uint32_t rank_cost(int len) {
-  return len > 0 ? (static_cast<uint32_t>(len) + kBN - 1) / kBN : 0u;
-}
 constexpr int kTablePages = 4096;  // page ids staged in LDS per workgroup (65536 keys)
+constexpr int kMergeRows = 32;     // rows of a segment-merge workgroup
+
+// An entry of the ranked work list.
+struct Work {
+  int seq, head, unit;  // unit: which of the (sequence, head)'s items
+  int row0, nq, len;    // the sequence's rows and keys
+  int n;                // its segments
+};
+
+// Items of one (sequence, head): a query tile of a segment each, or, for the
+// merge, kMergeRows rows of a cut sequence each.
+template <bool MERGE>
+__device__ __forceinline__ int seq_units(int nq, int n) {
+  if constexpr (MERGE) return n > 1 ? (nq + kMergeRows - 1) / kMergeRows : 0;
+  return (nq + kBM - 1) / kBM * n;
+}
+
+// Entry blockIdx.x of the ranked work list, by all 512 threads of a workgroup;
+// false past its end.  lds: 2 * kRankSeqs + 2 ints, free again on return.
+template <bool MERGE>
+__device__ __forceinline__ bool find_work(const PrefillArgs& a, void* lds, Work& w) {
+  // XCD b % 8 owns heads h == b % 8 (mod 8): hpx of them per sequence.
+  // Sequence s covers positions [hpx * before, hpx * (before + units)) of
+  // every XCD's queue, `before` being the units of the sequences ranked ahead.
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t max_len = a.width * kPage;
+  const int ns = a.num_seqs;
+  const int hpx = a.hq / kXcds;
+  const int xcd = static_cast<int>(blockIdx.x) % kXcds;
+  const int pos = static_cast<int>(blockIdx.x) / kXcds;
+  int before = 0;
+  if (ns <= kWaveSeqs) {
+    // One sequence per lane, every wave on its own: a memory round trip and
+    // kWaveSeqs steps in registers, no barrier.
+    const int s = min(lane, ns - 1);
+    int r0, nq;
+    seq_rows(a, s, r0, nq);
+    const int len = static_cast<int>(min<int64_t>(a.lens[s], max_len));
+    const int n = seq_segments(len, a.max_seg);
+    const int units = seq_units<MERGE>(nq, n);
+    const uint32_t key = static_cast<uint32_t>(segment_tiles(len, n)) * kWaveSeqs + (kWaveSeqs - 1 - s);
+    // Lanes past ns hold copies of the last sequence: q >= ns counts nothing.
+    const int mine = lane < ns ? units : 0;
+#pragma unroll
+    for (int q = 0; q < kWaveSeqs; ++q) {
+      const uint32_t kq = __builtin_amdgcn_readlane(key, q);
+      before += kq > key ? __builtin_amdgcn_readlane(mine, q) : 0;
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < ns && pos >= hpx * before && pos < hpx * (before + units));
+    if (hit == 0) return false;
+    w.seq = __builtin_ctzll(hit);
+    before = __builtin_amdgcn_readlane(before, w.seq);
+    w.row0 = __builtin_amdgcn_readlane(r0, w.seq);
+    w.nq = __builtin_amdgcn_readlane(nq, w.seq);
+    w.len = __builtin_amdgcn_readlane(len, w.seq);
+    w.n = __builtin_amdgcn_readlane(n, w.seq);
+  } else {
+    // One sequence per thread, costs and units exchanged through LDS.
+    uint32_t* s_key = static_cast<uint32_t*>(lds);             // [kRankSeqs] cost, then index
+    int* s_units = reinterpret_cast<int*>(s_key + kRankSeqs);  // [kRankSeqs]
+    int* s_hit = s_units + kRankSeqs;                          // the workgroup's sequence: index, before
+    int r0, nq = 0, len = 0, n = 1, units = 0;
+    uint32_t key = 0;
+    if (tid < ns) {
+      seq_rows(a, tid, r0, nq);
+      len = static_cast<int>(min<int64_t>(a.lens[tid], max_len));
+      n = seq_segments(len, a.max_seg);
+      units = seq_units<MERGE>(nq, n);
+      // 23 bits of cost: longer contexts (over 2^29 keys) rank by index.
+      const uint32_t cost = static_cast<uint32_t>(segment_tiles(len, n));
+      key = min(cost, (1u << 23) - 1) * kRankSeqs + (kRankSeqs - 1 - tid);
+    }
+    s_key[tid] = key;  // slots past ns count nothing
+    s_units[tid] = units;
+    if (tid == 0) s_hit[0] = -1;
+    __syncthreads();
+    if (tid < ns) {
+      for (int q = 0; q < ns; q += 16) {
+        u32x4 k4[4], u4[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          k4[i] = *reinterpret_cast<const u32x4*>(s_key + q + 4 * i);
+          u4[i] = *reinterpret_cast<const u32x4*>(s_units + q + 4 * i);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) before += k4[i][e] > key ? static_cast<int>(u4[i][e]) : 0;
+      }
+      if (pos >= hpx * before && pos < hpx * (before + units)) {
+        s_hit[0] = tid;
+        s_hit[1] = before;
+      }
+    }
+    __syncthreads();
+    w.seq = uniform(s_hit[0]);
+    if (w.seq < 0) return false;
+    before = uniform(s_hit[1]);
+    seq_rows(a, w.seq, r0, nq);
+    w.row0 = uniform(r0), w.nq = uniform(nq);
+    w.len = uniform(static_cast<int>(min<int64_t>(a.lens[w.seq], max_len)));
+    w.n = seq_segments(w.len, a.max_seg);
+    __syncthreads();  // the ranking arrays are dead before the caller reuses them
+  }
+  const int units = seq_units<MERGE>(w.nq, w.n);
+  const int local = pos - hpx * before;
+  w.head = xcd + kXcds * (local / units);
+  w.unit = local % units;
+  return true;
+}
 
 template <typename T, int D, bool DMA>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void paged_prefill_mfma_kernel(PrefillArgs a) {
@@ -210,90 +353,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   const int wave = uniform(tid >> 6);  // scalar, so per-wave conditions branch on SCC
   const int64_t max_len = a.width * kPage;
   int seq, t, h, row0, nq, len_k;
+  int nseg = 1, seg = 0;
   if (a.ranked) {
-    // XCD b % 8 owns heads h == b % 8 (mod 8): hpx of them per sequence.
-    // Sequence s covers positions [hpx * before, hpx * (before + qt)) of every
-    // XCD's queue, `before` being the query tiles of the sequences ranked
-    // ahead of it.
-    const int ns = a.num_seqs;
-    const int hpx = a.hq / kXcds;
-    const int xcd = static_cast<int>(blockIdx.x) % kXcds;
-    const int pos = static_cast<int>(blockIdx.x) / kXcds;
-    int before = 0, qt;
-    if (ns <= kWaveSeqs) {
-      // One sequence per lane, every wave on its own: a memory round trip and
-      // kWaveSeqs steps in registers, no barrier.
-      const int s = min(lane, ns - 1);
-      int r0, n;
-      seq_rows(a, s, r0, n);
-      const int len = static_cast<int>(min<int64_t>(a.lens[s], max_len));
-      const int tiles = (n + kBM - 1) / kBM;
-      const uint32_t key = rank_cost(len) * kWaveSeqs + (kWaveSeqs - 1 - s);
-      // Lanes past ns hold copies of the last sequence: q >= ns counts nothing.
-      const int mine = lane < ns ? tiles : 0;
-#pragma unroll
-      for (int q = 0; q < kWaveSeqs; ++q) {
-        const uint32_t kq = __builtin_amdgcn_readlane(key, q);
-        before += kq > key ? __builtin_amdgcn_readlane(mine, q) : 0;
-      }
-      const uint64_t hit =
-          __builtin_amdgcn_ballot_w64(lane < ns && pos >= hpx * before && pos < hpx * (before + tiles));
-      if (hit == 0) return;
-      seq = __builtin_ctzll(hit);
-      before = __builtin_amdgcn_readlane(before, seq);
-      qt = __builtin_amdgcn_readlane(tiles, seq);
-      row0 = __builtin_amdgcn_readlane(r0, seq);
-      nq = __builtin_amdgcn_readlane(n, seq);
-      len_k = __builtin_amdgcn_readlane(len, seq);
-    } else {
-      // One sequence per thread, costs and tiles exchanged through LDS.
-      uint32_t* s_key = reinterpret_cast<uint32_t*>(lds);        // [kRankSeqs] cost, then index
-      int* s_qt = reinterpret_cast<int*>(s_key + kRankSeqs);     // [kRankSeqs] query tiles
-      int* s_hit = s_qt + kRankSeqs;                             // the workgroup's sequence: index, before
-      int tiles = 0;
-      uint32_t key = 0;
-      if (tid < ns) {
-        int r0, n;
-        seq_rows(a, tid, r0, n);
-        tiles = (n + kBM - 1) / kBM;
-        // 23 bits of cost: longer contexts (over 2^29 keys) rank by index.
-        const uint32_t cost = rank_cost(static_cast<int>(min<int64_t>(a.lens[tid], max_len)));
-        key = min(cost, (1u << 23) - 1) * kRankSeqs + (kRankSeqs - 1 - tid);
-      }
-      s_key[tid] = key;  // slots past ns count nothing
-      s_qt[tid] = tiles;
-      if (tid == 0) s_hit[0] = -1;
-      __syncthreads();
-      if (tid < ns) {
-        for (int q = 0; q < ns; q += 16) {
-          u32x4 k4[4], w4[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            k4[i] = *reinterpret_cast<const u32x4*>(s_key + q + 4 * i);
-            w4[i] = *reinterpret_cast<const u32x4*>(s_qt + q + 4 * i);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) before += k4[i][e] > key ? static_cast<int>(w4[i][e]) : 0;
-        }
-        if (pos >= hpx * before && pos < hpx * (before + tiles)) {
-          s_hit[0] = tid;
-          s_hit[1] = before;
-        }
-      }
-      __syncthreads();
-      seq = uniform(s_hit[0]);
-      if (seq < 0) return;
-      before = uniform(s_hit[1]);
-      qt = uniform(s_qt[seq]);
-      seq_rows(a, seq, row0, nq);
-      len_k = static_cast<int>(min<int64_t>(a.lens[seq], max_len));
-      __syncthreads();  // the ranking arrays are dead before the tiles reuse them
-    }
-    const int local = pos - hpx * before;
-    h = xcd + kXcds * (local / qt);
-    t = qt - 1 - local % qt;
+    Work w;
+    if (!find_work<false>(a, lds, w)) return;
+    const int qt = (w.nq + kBM - 1) / kBM;
+    seq = w.seq, h = w.head, row0 = w.row0, nq = w.nq, len_k = w.len;
+    seg = w.unit / qt;
+    t = qt - 1 - (w.unit - seg * qt);
+    nseg = w.n;
   } else {
     const int w = blockIdx.x;
     h = w % a.hq;
@@ -307,14 +375,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   // Scalar from here on: the tile loop branches on them.
   seq = uniform(seq), t = uniform(t), h = uniform(h);
   row0 = uniform(row0), nq = uniform(nq), len_k = uniform(len_k);
+  nseg = uniform(nseg), seg = uniform(seg);
+  // The item's keys start at seg_key0; everything below counts from there.
+  const int seg_tiles = segment_tiles(len_k, nseg);
+  const int seg_key0 = seg * seg_tiles * kBN;
+  len_k -= seg_key0;
   const int prefix = len_k - nq;
   const int kvh = h / (a.hq / a.hkv);
   const int qt0 = t * kBM;                         // first chunk row of the workgroup
   const int wg_last_row = min(qt0 + kBM, nq) - 1;  // last chunk row of the workgroup
   const int wg_keys = prefix + wg_last_row + 1;    // <= len_k, so len_k >= 1 below
+  if (wg_keys <= 0 && seg > 0) return;             // the merge skips a segment past the tile's keys
   if (wg_keys <= 0) {
     // No row of the tile sees a key (a context shorter than its chunk): the
-    // rows are written as zeros, as a row that sees no key is below.
+    // rows are written as zeros, as a row that sees no key is below, and the
+    // merge leaves them alone.
     constexpr int CH = D / 8;  // 16-byte chunks per row
     const int rows = wg_last_row + 1 - qt0;
     for (int i = tid; i < rows * CH; i += 512) {
@@ -323,7 +398,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
     }
     return;
   }
-  const int ntiles = (wg_keys + kBN - 1) / kBN;
+  const int ntiles = min((wg_keys + kBN - 1) / kBN, seg_tiles);
 
   // Waves 0-3 take key tiles 0, 2, 4, ...; waves 4-7 tiles 1, 3, 5, ...; wave
   // w and w + 4 own the same 32 query rows and merge at the end.
@@ -355,7 +430,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   // time (one per lane, a chunk ahead of use) and are picked with readlane.
   // Slots past the sequence's last key re-read its last key (masked, but
   // finite: no unwritten slot is read); out-of-range ids read block 0.
-  const int32_t* trow = a.tables + static_cast<int64_t>(seq) * a.table_stride;
+  const int32_t* trow = a.tables + static_cast<int64_t>(seq) * a.table_stride + seg_key0 / kPage;
   const char* kbase = static_cast<const char*>(a.k) + static_cast<int64_t>(kvh) * a.kv_head * sizeof(T);
   const char* vbase = static_cast<const char*>(a.v) + static_cast<int64_t>(kvh) * a.kv_head * sizeof(T);
   const int64_t block_bytes = a.kv_block * static_cast<int64_t>(sizeof(T));
@@ -842,9 +917,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   xml[wave * 64 + lane] = make_float2(m, lsum);
   __syncthreads();
   float total;  // the row's sum of P
+  float mm;     // its maximum
   {
     const float2 other = xml[(wave ^ 4) * 64 + lane];
-    const float mm = fmaxf(m, other.x);
+    mm = fmaxf(m, other.x);
     const float c0 = (m == -INFINITY) ? 0.f : fast_exp2(m - mm);
     const float c1 = (other.x == -INFINITY) ? 0.f : fast_exp2(other.x - mm);
     total = lsum * c0 + other.y * c1;
@@ -859,6 +935,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
       }
   }
   if (!wave_live) return;
+  if (nseg > 1) {
+    // A segment's partial: unnormalised, for the merge kernel.  A store
+    // instruction writes 16 bytes of 32 consecutive rows per half wave.
+    if constexpr (DMA) {
+      if (!row_valid) return;
+      const int64_t part = static_cast<int64_t>(h) * a.max_seg + seg;
+      auto* const dst = (__attribute__((address_space(1))) f32x4*)a.part_acc +
+                        (part * (D / 4) + kg * 8 * HT + half) * a.total_q + row0 + my_row;
+#pragma unroll
+      for (int c = 0; c < HT; ++c)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          dst[static_cast<int64_t>(c * 8 + g * 2) * a.total_q] =
+              f32x4{keep[c][4 * g], keep[c][4 * g + 1], keep[c][4 * g + 2], keep[c][4 * g + 3]};
+      if (kg == 0 && half == 0) a.part_ml[part * a.total_q + row0 + my_row] = make_float2(mm, total);
+    }
+    return;
+  }
   // Through the wave's own LDS rows, so that a store instruction writes whole
   // runs of a row's half (16 bytes per lane) instead of 8 bytes of 32 rows.
   const float inv = total > 0.f ? 1.f / total : 0.f;  // a row that sees no key is written as zeros
@@ -882,6 +976,85 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
   }
 }
 
+// Merges the segment partials of kMergeRows rows of one (cut sequence, head):
+// out = sum_g acc_g 2^(m_g - M) / sum_g l_g 2^(m_g - M), segments in order.
+// A chain of memory round trips rather than bytes (520 per row, head and
+// segment): the first batch of accumulators goes out with the (max, sum) of
+// every segment, before any of them is known, and the rows leave through LDS
+// in whole 256-byte runs.  A row's later segments that start past its query
+// tile's last key were not computed and are not used.
+template <typename T>
+__global__ __launch_bounds__(512) void paged_prefill_merge_kernel(PrefillArgs a) {
+  using Ops = MfmaOps<T>;
+  constexpr int D = 128, QUADS = D / 4;
+  constexpr int QPT = QUADS * kMergeRows / 512;  // quads per thread
+  constexpr int QSTEP = 512 / kMergeRows;
+  constexpr int OROW = D + 8;  // padded output rows, elements
+  constexpr int kBatch = 8;    // segments in flight
+  __shared__ __align__(16) uint16_t rows[kMergeRows * OROW];
+  static_assert((2 * kRankSeqs + 2) * 4 <= kMergeRows * OROW * 2 && kBM % kMergeRows == 0, "ranking fits");
+  Work w;
+  if (!find_work<true>(a, rows, w)) return;
+  const int tid = threadIdx.x;
+  const int row0 = w.unit * kMergeRows;
+  const int r = tid % kMergeRows, q0 = tid / kMergeRows;
+  const int row = w.row0 + min(row0 + r, w.nq - 1);  // past the chunk: its last row, not stored
+  // Segments of this query tile: those that start before its last key.
+  const int tile_last = min(row0 / kBM * kBM + kBM, w.nq) - 1;
+  const int tile_keys = w.len - w.nq + tile_last + 1;
+  if (tile_keys <= 0) return;  // written as zeros already
+  const int seg_keys = segment_tiles(w.len, w.n) * kBN;
+  const int live = min(w.n, (tile_keys + seg_keys - 1) / seg_keys);
+  const int64_t part = static_cast<int64_t>(w.head) * a.max_seg;
+  float2 ml[kMaxSeg];
+#pragma unroll
+  for (int g = 0; g < kMaxSeg; ++g) ml[g] = a.part_ml[(part + min(g, live - 1)) * a.total_q + row];
+  f32x4 x[kBatch][QPT];
+  auto load = [&](int g0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+      for (int i = 0; i < QPT; ++i)
+        x[u][i] = a.part_acc[((part + min(g0 + u, live - 1)) * QUADS + q0 + i * QSTEP) * a.total_q + row];
+  };
+  load(0);
+  float M = -INFINITY;
+#pragma unroll
+  for (int g = 0; g < kMaxSeg; ++g) M = fmaxf(M, ml[g].x);  // copies of the last segment change nothing
+  float acc[QPT][4] = {};
+  float sum = 0.f;
+#pragma unroll
+  for (int g0 = 0; g0 < kMaxSeg; g0 += kBatch) {
+    if (g0 >= live) break;
+    if (g0 > 0) load(g0);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const bool on = g0 + u < live && ml[g0 + u].x != -INFINITY;
+      const float f = on ? fast_exp2(ml[g0 + u].x - M) : 0.f;
+      sum = on ? fmaf(ml[g0 + u].y, f, sum) : sum;
+#pragma unroll
+      for (int i = 0; i < QPT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = on ? fmaf(x[u][i][e], f, acc[i][e]) : acc[i][e];
+    }
+  }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;  // a row that sees no key is written as zeros
+#pragma unroll
+  for (int i = 0; i < QPT; ++i) {
+    const u32x2 v = {Ops::pack2(acc[i][0] * inv, acc[i][1] * inv), Ops::pack2(acc[i][2] * inv, acc[i][3] * inv)};
+    *reinterpret_cast<u32x2*>(rows + r * OROW + (q0 + i * QSTEP) * 4) = v;
+  }
+  __syncthreads();
+  constexpr int OCH = D / 8;  // 16-byte chunks per row
+  T* const obase = static_cast<T*>(a.out) + (static_cast<int64_t>(w.row0) + row0) * a.o_row +
+                   static_cast<int64_t>(w.head) * a.o_head;
+  for (int i = tid; i < kMergeRows * OCH; i += 512) {
+    const int rr = i / OCH, c = i % OCH;
+    if (row0 + rr < w.nq)
+      *reinterpret_cast<u32x4*>(obase + rr * a.o_row + c * 8) = *reinterpret_cast<const u32x4*>(rows + rr * OROW + c * 8);
+  }
+}
+
 int64_t expand_bytes(int64_t total_q, int64_t width) {
   const int64_t lens = (total_q * 4 + 255) / 256 * 256;
   const int64_t tables = (total_q * std::max<int64_t>(width, 1) * 4 + 255) / 256 * 256;
@@ -900,6 +1073,24 @@ namespace {
 bool mfma_shape(int64_t head_dim, int64_t page_size, int dtype) {
   return (dtype == RLT_BFLOAT16 || dtype == RLT_FLOAT16) && (head_dim == 64 || head_dim == 128) && page_size == kPage;
 }
+// Segments a launch of these shapes allows its sequences (see kSegTiles): as
+// many as bring its query tiles, at least one per sequence, to one item per
+// CU.  1 when the direct-to-LDS kernel's work list is not the ranked one.
+int max_segments(int64_t total_q, int64_t num_seqs, int64_t width, int64_t hq) {
+  if (num_seqs > kRankSeqs || hq % kXcds || width > kTablePages) return 1;
+  const int64_t items = std::max<int64_t>((total_q + kBM - 1) / kBM, num_seqs) * hq;
+  const int64_t by_keys = width * kPage / kBN / kSegTiles;
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({kCus / items, by_keys, kMaxSeg})));
+}
+struct SplitLayout {
+  int64_t ml, total;  // the accumulators come first
+};
+SplitLayout split_layout(int64_t total_q, int64_t hq, int64_t d, int max_seg) {
+  if (max_seg <= 1) return {0, 0};
+  const int64_t slots = total_q * hq * max_seg;
+  const int64_t acc = (slots * d * 4 + 255) / 256 * 256;
+  return {acc, acc + (slots * 8 + 255) / 256 * 256};
+}
 int64_t fallback_workspace(int64_t total_q, int64_t width, int64_t hq, int64_t hkv, int64_t d) {
   return expand_bytes(total_q, width) + rlt_paged_decode_workspace_bytes(total_q, hq, hkv, d);
 }
@@ -914,13 +1105,24 @@ extern "C" int64_t rlt_paged_prefill_workspace_bytes(int64_t total_q, int64_t nu
   return fallback_workspace(total_q, max_table_width, num_q_heads, num_kv_heads, head_dim);
 }
 
-extern "C" int rlt_paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache,
-                                 const void* value_cache, const int64_t* kv_strides, const int32_t* block_tables,
-                                 int64_t table_stride, int64_t max_table_width, const int32_t* context_lengths,
-                                 const int32_t* cu_seqlens_q, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
-                                 void* out, const int64_t* out_strides, int64_t num_q_heads, int64_t num_kv_heads,
-                                 int64_t head_dim, int64_t page_size, int64_t num_blocks, float scale, int dtype,
-                                 void* workspace, int64_t workspace_bytes, void* stream) {
+extern "C" int64_t rlt_paged_prefill_split_workspace_bytes(int64_t total_q, int64_t num_seqs, int64_t max_table_width,
+                                                           int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
+                                                           int64_t page_size, int dtype) {
+  if (total_q <= 0 || num_seqs <= 0) return 0;
+  if (!mfma_shape(head_dim, page_size, dtype))
+    return fallback_workspace(total_q, max_table_width, num_q_heads, num_kv_heads, head_dim);
+  if (num_q_heads <= 0 || max_table_width <= 0 || head_dim != 128) return 0;
+  return split_layout(total_q, num_q_heads, head_dim, max_segments(total_q, num_seqs, max_table_width, num_q_heads)).total;
+}
+
+namespace {
+
+int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache, const void* value_cache,
+                  const int64_t* kv_strides, const int32_t* block_tables, int64_t table_stride, int64_t max_table_width,
+                  const int32_t* context_lengths, const int32_t* cu_seqlens_q, int64_t num_seqs, int64_t total_q,
+                  int64_t max_seqlen_q, void* out, const int64_t* out_strides, int64_t num_q_heads,
+                  int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_blocks, float scale, int dtype,
+                  void* workspace, int64_t workspace_bytes, void* stream, bool split) {
   if (!dtype_size(dtype)) return fail(RLT_EINVAL, "rlt_paged_prefill: unknown dtype %d", dtype);
   if (num_seqs < 0 || total_q < 0 || max_seqlen_q < 0)
     return fail(RLT_EINVAL, "rlt_paged_prefill: negative sizes");
@@ -982,15 +1184,24 @@ extern "C" int rlt_paged_prefill(const void* q, const int64_t* q_strides, const 
     if (!p.ranked && max_seqlen_q <= 0)
       return fail(RLT_EINVAL, "rlt_paged_prefill: max_seqlen_q must cover the longest chunk");
     p.max_qt = static_cast<int>(std::min<int64_t>(max_qt, 0x7fffffff));
-    const int64_t items = p.ranked ? pairs_bound * num_q_heads : num_seqs * max_qt * num_q_heads;
+    // Direct-to-LDS staging needs the key range's page ids to fit in LDS (and
+    // a workgroup's query rows within 32-bit offsets).
+    const bool dma = head_dim == 128 && max_table_width <= kTablePages && q_strides[0] >= 0 &&
+                     q_strides[0] * esize * kBM < (int64_t(1) << 31);
+    // Key segments, when the caller gave room for their partials.
+    p.max_seg = split && dma && p.ranked ? max_segments(total_q, num_seqs, max_table_width, num_q_heads) : 1;
+    const SplitLayout layout = split_layout(total_q, num_q_heads, head_dim, p.max_seg);
+    if (p.max_seg > 1 && workspace && aligned16(workspace) && workspace_bytes >= layout.total) {
+      p.part_acc = static_cast<f32x4*>(workspace);
+      p.part_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + layout.ml);
+    } else {
+      p.max_seg = 1;
+    }
+    const int64_t items = p.ranked ? pairs_bound * p.max_seg * num_q_heads : num_seqs * max_qt * num_q_heads;
     if (items > 0x7fffffff) return fail(RLT_EUNSUPPORTED, "rlt_paged_prefill: too many query tiles");
     if (items == 0) return RLT_OK;
     const dim3 grid(static_cast<unsigned>(items));
     hipStream_t st = as_stream(stream);
-    // Direct-to-LDS staging needs the key range's page ids to fit in LDS.
-    // (and a workgroup's query rows within 32-bit offsets).
-    const bool dma = head_dim == 128 && max_table_width <= kTablePages && q_strides[0] >= 0 &&
-                     q_strides[0] * esize * kBM < (int64_t(1) << 31);
     if (dtype == RLT_BFLOAT16) {
       if (dma) hipLaunchKernelGGL((paged_prefill_mfma_kernel<bf16, 128, true>), grid, dim3(512), 0, st, p);
       else if (head_dim == 128) hipLaunchKernelGGL((paged_prefill_mfma_kernel<bf16, 128, false>), grid, dim3(512), 0, st, p);
@@ -1000,7 +1211,12 @@ extern "C" int rlt_paged_prefill(const void* q, const int64_t* q_strides, const 
       else if (head_dim == 128) hipLaunchKernelGGL((paged_prefill_mfma_kernel<f16, 128, false>), grid, dim3(512), 0, st, p);
       else hipLaunchKernelGGL((paged_prefill_mfma_kernel<f16, 64, false>), grid, dim3(512), 0, st, p);
     }
-    return check_launch("rlt_paged_prefill");
+    if (p.max_seg == 1) return check_launch("rlt_paged_prefill");
+    if (int rc = check_launch("rlt_paged_prefill")) return rc;
+    const dim3 mgrid(static_cast<unsigned>(pairs_bound * (kBM / kMergeRows) * num_q_heads));
+    if (dtype == RLT_BFLOAT16) hipLaunchKernelGGL(paged_prefill_merge_kernel<bf16>, mgrid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL(paged_prefill_merge_kernel<f16>, mgrid, dim3(512), 0, st, p);
+    return check_launch("rlt_paged_prefill(merge)");
   }
 
   const int64_t need = fallback_workspace(total_q, max_table_width, num_q_heads, num_kv_heads, head_dim);
@@ -1028,4 +1244,32 @@ extern "C" int rlt_paged_prefill(const void* q, const int64_t* q_strides, const 
                           e.row_lens, out, out_strides, total_q, num_q_heads, num_kv_heads, head_dim, page_size,
                           num_blocks, scale, dtype, decode_ws, workspace_bytes - expand_bytes(total_q, max_table_width),
                           stream);
+}
+
+}  // namespace
+
+extern "C" int rlt_paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache,
+                                 const void* value_cache, const int64_t* kv_strides, const int32_t* block_tables,
+                                 int64_t table_stride, int64_t max_table_width, const int32_t* context_lengths,
+                                 const int32_t* cu_seqlens_q, int64_t num_seqs, int64_t total_q, int64_t max_seqlen_q,
+                                 void* out, const int64_t* out_strides, int64_t num_q_heads, int64_t num_kv_heads,
+                                 int64_t head_dim, int64_t page_size, int64_t num_blocks, float scale, int dtype,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
+  return paged_prefill(q, q_strides, key_cache, value_cache, kv_strides, block_tables, table_stride, max_table_width,
+                       context_lengths, cu_seqlens_q, num_seqs, total_q, max_seqlen_q, out, out_strides, num_q_heads,
+                       num_kv_heads, head_dim, page_size, num_blocks, scale, dtype, workspace, workspace_bytes, stream,
+                       false);
+}
+
+extern "C" int rlt_paged_prefill_split(const void* q, const int64_t* q_strides, const void* key_cache,
+                                       const void* value_cache, const int64_t* kv_strides, const int32_t* block_tables,
+                                       int64_t table_stride, int64_t max_table_width, const int32_t* context_lengths,
+                                       const int32_t* cu_seqlens_q, int64_t num_seqs, int64_t total_q,
+                                       int64_t max_seqlen_q, void* out, const int64_t* out_strides, int64_t num_q_heads,
+                                       int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_blocks,
+                                       float scale, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return paged_prefill(q, q_strides, key_cache, value_cache, kv_strides, block_tables, table_stride, max_table_width,
+                       context_lengths, cu_seqlens_q, num_seqs, total_q, max_seqlen_q, out, out_strides, num_q_heads,
+                       num_kv_heads, head_dim, page_size, num_blocks, scale, dtype, workspace, workspace_bytes, stream,
+                       true);
 }

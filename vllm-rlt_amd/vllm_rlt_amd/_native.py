@@ -103,6 +103,15 @@ SIGNATURES = {
         + [c_int64] * 5
         + [c_float, c_int, c_void_p, c_int64, c_void_p],
     ),
+    "rlt_paged_prefill_split_workspace_bytes": (c_int64, [c_int64] * 7 + [c_int]),
+    "rlt_paged_prefill_split": (
+        c_int,
+        [c_void_p, _i64p, c_void_p, c_void_p, _i64p, c_void_p, c_int64, c_int64, c_void_p, c_void_p]
+        + [c_int64] * 3
+        + [c_void_p, _i64p]
+        + [c_int64] * 5
+        + [c_float, c_int, c_void_p, c_int64, c_void_p],
+    ),
     "rlt_kv_finalize": (
         c_int,
         [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, _i64p]

@@ -268,6 +268,18 @@ def prefill_workspace_bytes(
     )
 
 
+def prefill_split_workspace_bytes(
+    total_q: int, num_seqs: int, table_width: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
+    page_size: int, dtype: torch.dtype,
+) -> int:
+    """Bytes rlt_paged_prefill_split needs: the partials of cut key ranges on the MFMA path, else the per-token path's."""
+    return int(
+        _native.load().rlt_paged_prefill_split_workspace_bytes(
+            total_q, num_seqs, table_width, num_q_heads, num_kv_heads, head_dim, page_size, dtype_code(dtype)
+        )
+    )
+
+
 # rlt_paged_decode's split plan: rows are cut into splits of 256 tokens, and
 # a row needing more than 64 splits doubles the split length until 64 cover it.
 DECODE_SPLIT_TOKENS = 256
@@ -581,8 +593,20 @@ def paged_prefill(
     The MFMA path needs no workspace; other shapes (fp32, unaligned rows,
     other head sizes) run each query row as a decode row and need
     prefill_workspace_bytes(...) bytes, allocated here unless `workspace`
-    (a uint8 device tensor at least that large) is given.
+    (a uint8 device tensor at least that large) is given.  Without a given
+    workspace, long key ranges of short chunks are cut into segments whose
+    partials are allocated here (rlt_paged_prefill_split).
     """
+    return _paged_prefill(
+        q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace,
+        workspace is None,
+    )
+
+
+def _paged_prefill(
+    q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace, split
+):
+    """paged_prefill; split: the workspace is this call's alone, so segment partials may go there."""
     device = _require_rocm(q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q)
     if q.ndim != 3 or key_cache.ndim != 4:
         raise ValueError("q must be [tokens, heads, head_dim] and caches [blocks, page, kv_heads, head_dim]")
@@ -612,13 +636,14 @@ def paged_prefill(
     code = dtype_code(q.dtype)
     if not all(_rows_aligned16(t) for t in (q, out, key_cache, value_cache)):
         code = _native.RLT_FLOAT32  # the MFMA path needs 16-byte rows; size the per-token fallback
-    need = int(lib.rlt_paged_prefill_workspace_bytes(total, nseq, width, hq, hkv, d, page, code))
+    size_of = lib.rlt_paged_prefill_split_workspace_bytes if split else lib.rlt_paged_prefill_workspace_bytes
+    need = int(size_of(total, nseq, width, hq, hkv, d, page, code))
     if workspace is None:
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
     elif workspace.numel() * workspace.element_size() < need or workspace.device != device:
         raise ValueError(f"workspace must hold {need} bytes on {device}")
     scale = 1.0 / math.sqrt(d) if scale is None else scale
-    rc = lib.rlt_paged_prefill(
+    rc = (lib.rlt_paged_prefill_split if split else lib.rlt_paged_prefill)(
         q.data_ptr(),
         int64_array(q.stride()),
         key_cache.data_ptr(),
