@@ -1,0 +1,78 @@
+"""Decode items by one wave and by four: the same bits, and the oracle's result (GPU).
+
+A split's tokens are kept in quarters; small launches give every quarter a
+wave, larger ones walk them with one.  Lengths sit at the edges of tiles (32),
+quarters (64) and splits (256).
+"""
+
+import pytest
+import torch
+
+from oracle.paged_attention import paged_attention_cpu
+from paged_cases import random_decode_case
+from test_decode_gpu import TOL
+
+pytestmark = pytest.mark.gpu
+
+ONE_SPLIT = [0, 1, 16, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129, 161, 191, 192, 193, 224, 255, 256]
+LONGER = ONE_SPLIT + [257, 288, 320, 321, 447, 511, 512, 513, 705, 1000]
+# Past 64 splits of 256 tokens a split, and with it a quarter, doubles.
+LONG = [16384, 16385, 16640, 17000]
+
+
+def by_row(run, case, append):
+    """Each row of the case in a launch of its own."""
+    outs = []
+    for r in range(len(case.lengths)):
+        outs.append(run(case, slice(r, r + 1), append))
+    return torch.cat(outs)
+
+
+def launch(case, rows, append):
+    from vllm_rlt_amd import ops
+
+    q, tables, lengths = case.q[rows], case.tables[rows], case.lengths[rows]
+    if not append:
+        return ops.paged_decode(q, case.key_slice, case.value_slice, tables, lengths)
+    k, v, blocks, offsets = (t[rows] for t in append)
+    return ops.paged_decode_append(
+        q, case.key_slice, case.value_slice, tables, lengths, k.contiguous(), v.contiguous(), blocks.contiguous(),
+        offsets.contiguous(),
+    )
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lengths", [ONE_SPLIT, LONGER, LONG], ids=["one_split", "longer", "long"])
+def test_one_wave_and_four_give_the_same_bits(lengths, dtype, fused):
+    heads = 4 if lengths is LONG else 16
+    # Rows alone are small launches; the batch repeats them until it is a large one.
+    case = random_decode_case(lengths, hq=heads, hkv=heads, d=128, dtype=dtype, seed=len(lengths))
+    dev = case.to("cuda")
+    append = None
+    if fused:
+        last = (dev.lengths.long() - 1).clamp(min=0)
+        blocks = dev.tables[torch.arange(len(lengths), device="cuda"), last // 16].long()
+        blocks[dev.lengths == 0] = -1  # nowhere
+        # The new token is what the page already holds: every launch appends the same bytes.
+        safe = blocks.clamp(min=0)
+        append = (dev.key_slice[safe, last % 16], dev.value_slice[safe, last % 16], blocks, last % 16)
+    alone = by_row(launch, dev, append)
+    copies = max(1, 4200 // (heads * len(lengths)))
+    many = random_case_copies(dev, copies)
+    batch = launch(many, slice(None), tuple(t.repeat((copies,) + (1,) * (t.ndim - 1)) for t in append) if append else None)
+    torch.cuda.synchronize()
+    print(f"[decode quarters] {dtype} fused={fused} rows={len(lengths) * copies}", flush=True)
+    assert torch.equal(batch, alone.repeat(copies, 1, 1))
+    atol, rtol = TOL[dtype]
+    expect = paged_attention_cpu(case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
+    torch.testing.assert_close(alone.cpu(), expect, atol=atol, rtol=rtol)
+
+
+def random_case_copies(case, copies):
+    """The case with its rows repeated; the copies read the same pages."""
+    from dataclasses import replace
+
+    return replace(
+        case, q=case.q.repeat(copies, 1, 1), tables=case.tables.repeat(copies, 1), lengths=case.lengths.repeat(copies)
+    )

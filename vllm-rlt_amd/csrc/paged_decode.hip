@@ -89,6 +89,19 @@ constexpr int kMaxGrid = RLT_DECODE_MAX_GRID;
 #ifndef RLT_DECODE_XCD_SCHEDULE
 #define RLT_DECODE_XCD_SCHEDULE 1
 #endif
+// Launches of at most this many (row, kv head, split) items, splits counted
+// from the table width, give an item four waves: 2 waves per SIMD hold 2048
+// one-wave items at once, and below half of that the launch takes as long as
+// one item does.  Measured (16 heads, us, one wave against four): 4 rows of
+// 128-256 tokens 11.7 / 6.3, 1 of 256-512 13.9 / 9.3, 8 of 512-1024 18.0 /
+// 16.8 (640 items), 16 of 256-512 18.7 / 16.8 (768); 8 of 1024-2048 21.9 /
+// 25.5 (1152).  One-split launches of more than half as many only when the
+// table spans more than two quarters: 64 rows of 128-256 tokens 28.9 / 21.5,
+// of 32-64 11.4 / 13.3.
+#ifndef RLT_DECODE_QUAD_ITEMS
+#define RLT_DECODE_QUAD_ITEMS 1024
+#endif
+constexpr int kQuadItems = RLT_DECODE_QUAD_ITEMS;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, workgroups dispatched round-robin
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -383,6 +396,15 @@ __device__ void merge_partials(const DecodeArgs& a, int r, int h, int j, int ns,
   }
 }
 
+// Whether items keep their splits in quarters: where the quarter's and the
+// split's state fit the registers side by side without costing a wave per SIMD
+// (fp32 and head_dim 256 spill, two q heads per kv head drop from three waves
+// to two).
+template <typename T, int D, int G>
+constexpr bool quarters() {
+  return G == 1 && D == 128 && sizeof(T) == 2;
+}
+
 // The prefix pass's work item (defined with the prefix pass below).
 template <typename T, int G>
 __device__ __forceinline__ void shared_prefix_item(const DecodeArgs& a, int item, int h, uint16_t* tiles);
@@ -392,7 +414,10 @@ __device__ __forceinline__ void shared_prefix_item(const DecodeArgs& a, int item
 // row is a single split (the tables span at most one split), so each row's one
 // item stores the row's new token itself (APPEND), after its own reads, and no
 // merge kernel runs.
-template <typename T, int D, int G, int P, int TILE, bool XCD, bool PREFIX, bool APPEND, bool ONE_SPLIT = false>
+// QUAD: the workgroup's four waves share one item, a quarter of its tokens
+// each (see kQuarters).
+template <typename T, int D, int G, int P, int TILE, bool XCD, bool PREFIX, bool APPEND, bool ONE_SPLIT = false,
+          bool QUAD = false>
 __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const int blocks) {
   using PK = Packet<T>;
   constexpr int EPL = PK::N;      // elements of one token a lane owns
@@ -409,6 +434,14 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   const int g = lane / LPT;
   const int s = lane % LPT;
   const uint32_t lane_dim = static_cast<uint32_t>(s * EPL);
+  // Items (quarters<T, D, G>) keep a quarter's softmax state and
+  // fold it into the split's at the quarter's end (fold below), in this order
+  // in every launch: so one wave that walks the quarters and four waves that
+  // take one each give the same bits, and the host may choose by the launch.
+  constexpr bool kQuarters = quarters<T, D, G>();
+  static_assert(!QUAD || (kQuarters && XCD && !PREFIX), "shared items");
+  constexpr int kStateFloats = G * (EPL + 2);
+  __shared__ float quarter_state[QUAD ? (kWaves - 1) * kStateFloats * 64 : 1];
 
   // A one-split launch's append: row r's new token of kv head h into its
   // write slot (skipped when the slot is outside the pool), by the lanes of
@@ -428,9 +461,12 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     }
   };
 
-  // One (row r, kv head h, split sp) item per wave.
-  auto process = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns) {
+  // One (row r, kv head h, split sp) item per wave (per workgroup: QUAD).
+  // first_entry: QUAD's page ids of this wave's first 64 pages when early.
+  auto process = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns,
+                     const bool early = false, const int first_entry = 0) {
     if (len <= 0) {
+      if (QUAD && wave != 0) return;
       if (g == 0) {
         T* orow = static_cast<T*>(a.out) + r * a.o_row + static_cast<int64_t>(h) * G * a.o_head + lane_dim;
         const u32x4 zero = {0u, 0u, 0u, 0u};
@@ -440,8 +476,9 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       store_new_token(r, h);
       return;
     }
-    const int t_begin = sp * split_len;
-    const int t_end = min(len, t_begin + split_len);
+    const int quarter = split_len / kWaves;
+    const int t_begin = sp * split_len + (QUAD ? wave * quarter : 0);
+    const int t_end = min(len, t_begin + (QUAD ? quarter : split_len));
     const int last = t_end - 1;
     // Fused append: the row's write slot, read up front when this is its last split.
     int64_t wb = -1, wo = -1;
@@ -466,13 +503,59 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     }
 
     float m[G], l[G], acc[G][EPL];
+    auto reset = [&]() {
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
-      m[j] = -INFINITY;
-      l[j] = 0.f;
+      for (int j = 0; j < G; ++j) {
+        m[j] = -INFINITY;
+        l[j] = 0.f;
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) acc[j][e] = 0.f;
+        for (int e = 0; e < EPL; ++e) acc[j][e] = 0.f;
+      }
+    };
+    reset();
+    // The split's state, and a quarter's (qm, ql, qa) folded into it; written
+    // out with fmaf so that every kernel rounds alike.
+    float sm[G], sl[G], sa[G][EPL];
+    if constexpr (kQuarters) {
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        sm[j] = -INFINITY;
+        sl[j] = 0.f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) sa[j][e] = 0.f;
+      }
     }
+    auto fold = [&](const float (&qm)[G], const float (&ql)[G], const float (&qa)[G][EPL]) {
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const float mn = fmaxf(sm[j], qm[j]);
+        const float fs = sm[j] == -INFINITY ? 0.f : fast_exp2(sm[j] - mn);
+        const float fq = qm[j] == -INFINITY ? 0.f : fast_exp2(qm[j] - mn);
+        sl[j] = fmaf(sl[j], fs, ql[j] * fq);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) sa[j][e] = fmaf(sa[j][e], fs, qa[j][e] * fq);
+        sm[j] = mn;
+      }
+    };
+    // One wave walking all quarters: after the tile that ends one.
+    auto end_tile = [&](int t0) {
+      if constexpr (kQuarters && !QUAD) {
+        if (((t0 + TILE - t_begin) & (quarter - 1)) == 0 || t0 + TILE >= t_end) {
+          if (t0 - t_begin < quarter) {  // the first quarter: folding it into nothing is a copy
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+              sm[j] = m[j];
+              sl[j] = l[j];
+#pragma unroll
+              for (int e = 0; e < EPL; ++e) sa[j][e] = acc[j][e];
+            }
+          } else {
+            fold(m, l, acc);
+          }
+          reset();
+        }
+      }
+    };
 
     const int32_t* trow = a.tables + r * a.table_stride;
     const T* kbase = static_cast<const T*>(a.k) + static_cast<int64_t>(h) * a.kv_head;
@@ -537,7 +620,9 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       const int c1 = min(t_end, c0 + kChunkTokens);
       const int chunk_page = c0 / P;
       const int chunk_last = (c1 - 1) / P - chunk_page;  // <= 63
-      const int table_entry = lane <= chunk_last ? trow[chunk_page + lane] : 0;
+      int table_entry;
+      if (QUAD && early) table_entry = first_entry;  // a quarter is one chunk then
+      else table_entry = lane <= chunk_last ? trow[chunk_page + lane] : 0;
       auto tile_pages = [&](int t0, int64_t (&blk)[PPT]) {
         const int rel0 = (t0 - c0) / P;
 #pragma unroll
@@ -590,6 +675,34 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       }
       u32x4 kp[NI], vp[NI];
       int64_t blk[PPT];
+      if constexpr (QUAD) {
+        if (quarter == 2 * TILE) {
+          // Both tiles of a 64-token quarter in flight at once.  A second tile
+          // past the end re-reads the last token and adds exactly nothing.
+          u32x4 kp2[NI], vp2[NI];
+          int64_t blk2[PPT];
+          tile_pages(c0, blk);
+          tile_pages(c0 + TILE, blk2);
+          if (APPEND && fresh) {
+            issue_fresh(kp, kbase, kn_row, blk, c0);
+            issue_fresh(kp2, kbase, kn_row, blk2, c0 + TILE);
+            issue_fresh(vp, vbase, vn_row, blk, c0);
+            issue_fresh(vp2, vbase, vn_row, blk2, c0 + TILE);
+          } else {
+            issue(kp, kbase, blk, c0);
+            issue(kp2, kbase, blk2, c0 + TILE);
+            issue(vp, vbase, blk, c0);
+            issue(vp2, vbase, blk2, c0 + TILE);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          float sc[G][NI];
+          scores(kp, c0, sc);
+          accumulate(vp, c0, sc);
+          scores(kp2, c0 + TILE, sc);
+          accumulate(vp2, c0 + TILE, sc);
+          continue;
+        }
+      }
       // sched_barrier keeps every K load of a tile ahead of its V loads in
       // issue order, so waiting for K never waits for V.
       tile_pages(c0, blk);
@@ -614,6 +727,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
         accumulate(vp, t0, sc);
         issue(vp, vbase, blk, t0 + TILE);
         __builtin_amdgcn_sched_barrier(0);
+        end_tile(t0);
       }
       if constexpr (APPEND) {
         if (fresh && ntiles > 1) {
@@ -625,12 +739,51 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
           accumulate(vp, t0, sc);
           issue_fresh(vp, vbase, vn_row, blk, t0 + TILE);
           __builtin_amdgcn_sched_barrier(0);
+          end_tile(t0);
           t0 += TILE;
         }
       }
       float sc[G][NI];
       scores(kp, t0, sc);
       accumulate(vp, t0, sc);
+      end_tile(t0);
+    }
+    if constexpr (QUAD) {
+      // Wave 0 folds the quarters in order; the others hand theirs over.
+      float* const mine = quarter_state + (wave - 1) * kStateFloats * 64 + lane;
+      if (wave > 0) {
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+          mine[(j * (EPL + 2)) * 64] = m[j];
+          mine[(j * (EPL + 2) + 1) * 64] = l[j];
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) mine[(j * (EPL + 2) + 2 + e) * 64] = acc[j][e];
+        }
+      }
+      __syncthreads();  // and every read of the item's pages is done
+      if (wave > 0) return;
+      fold(m, l, acc);
+#pragma unroll
+      for (int w = 0; w < kWaves - 1; ++w) {
+        const float* const q = quarter_state + w * kStateFloats * 64 + lane;
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+          m[j] = q[(j * (EPL + 2)) * 64];
+          l[j] = q[(j * (EPL + 2) + 1) * 64];
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) acc[j][e] = q[(j * (EPL + 2) + 2 + e) * 64];
+        }
+        fold(m, l, acc);
+      }
+    }
+    if constexpr (kQuarters) {
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        m[j] = sm[j];
+        l[j] = sl[j];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[j][e] = sa[j][e];
+      }
     }
 
     // Merge the token groups (lanes that share s).
@@ -901,6 +1054,28 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       if (ns == 1) store_new_token(r, h);
     }
   };
+  if constexpr (QUAD) {
+    // One (row, split, head) per workgroup, laid out as the XCD-affine
+    // schedule below with heads in place of head blocks.  The row's length,
+    // its page ids, and (in process) q and the write slot go out together when
+    // the split length does not depend on the row's own.
+    const int t = block / kXcds;
+    const int r = t % a.n_rows;
+    const int round = t / a.n_rows;
+    const int gi = kXcds * round + (block % kXcds + kXcds - round % kXcds) % kXcds;
+    if (gi >= a.xcd_groups) return;
+    const int sp = gi / a.hkv;
+    const int h = gi - sp * a.hkv;
+    const bool early = a.max_len <= kMaxSplits * kSplitTokens;
+    const int page0 = sp * (kSplitTokens / P) + wave * (kSplitTokens / P / kWaves);
+    const int width = static_cast<int>(a.max_len / P);
+    const int entry = early && width > 0 ? a.tables[r * a.table_stride + min(page0 + (lane & 3), width - 1)] : 0;
+    const int len = uniform(row_length(a, r));
+    int split_len, ns;
+    split_plan(len, &split_len, &ns);
+    if (sp < ns) process(r, h, sp, len, split_len, ns, early, entry);
+    return;
+  }
   auto run_item = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns) {
     if constexpr (kMfma) process_mfma(r, h, sp, len, split_len, ns);
     else process(r, h, sp, len, split_len, ns);
@@ -949,8 +1124,19 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   }
 }
 
+// Four waves to an item (quarters<T, D, G> only), for launches that leave most of
+// the chip idle.
+template <typename T, int D, int G, int P, int TILE, bool APPEND, bool ONE_SPLIT>
+__global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a) {
+  split_pass<T, D, G, P, TILE, true, false, APPEND, ONE_SPLIT, true>(a, blockIdx.x, gridDim.x);
+}
+
+// Items with quarters would fit three waves per SIMD (142 VGPRs), which streams
+// more slowly than two (64 rows of 512-4096 tokens 194.5 against 192.5 us, 256
+// of 1024-8192 1533 against 1527 us): naming v169 holds the kernel at two.
 template <typename T, int D, int G, int P, int TILE, bool XCD, bool APPEND, bool ONE_SPLIT>
 __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
+  if constexpr (quarters<T, D, G>() && !ONE_SPLIT) asm volatile("" ::: "v169");
   split_pass<T, D, G, P, TILE, XCD, false, APPEND, ONE_SPLIT>(a, blockIdx.x, gridDim.x);
 }
 
@@ -1358,6 +1544,18 @@ DecodeKernel pick_group(int G) {
   }
 }
 
+// The kernel that gives an item four waves, null where items have no quarters.
+template <typename T>
+DecodeKernel pick_quad(int d, int G, bool append, bool one_split) {
+  if constexpr (quarters<T, 128, 1>()) {
+    if (d != 128 || G != 1) return nullptr;
+    if (!append) return paged_decode_quad_kernel<T, 128, 1, 16, kTile, false, false>;
+    return one_split ? paged_decode_quad_kernel<T, 128, 1, 16, kTile, true, true>
+                     : paged_decode_quad_kernel<T, 128, 1, 16, kTile, true, false>;
+  }
+  return nullptr;
+}
+
 // The fused-append split pass is compiled for the XCD-affine schedule (with
 // and without the shared-prefix check); other cases append first, then decode.
 template <typename T, int D, bool PREFIX>
@@ -1484,7 +1682,15 @@ int launch_decode(DecodeArgs a, int64_t max_table_width, hipStream_t stream) {
     return check_launch("rlt_paged_decode(generic)");
   }
   const int64_t splits_cap = std::min<int64_t>(kMaxSplits, (max_tokens + kSplitTokens - 1) / kSplitTokens);
-  if (xcd) {
+  const int64_t items_bound = static_cast<int64_t>(a.n_rows) * a.hkv * std::max<int64_t>(splits_cap, 1);
+  const bool few = items_bound <= (single_split && max_tokens <= kSplitTokens / 2 ? kQuadItems / 2 : kQuadItems);
+  const DecodeKernel quad = xcd && !prefix && few ? pick_quad<T>(a.d, G, append, single_split) : nullptr;
+  if (quad) {
+    const int64_t groups = std::max<int64_t>(splits_cap, 1) * a.hkv;
+    const int64_t grid = static_cast<int64_t>(kXcds) * a.n_rows * ((groups + kXcds - 1) / kXcds);
+    a.xcd_groups = static_cast<int>(groups);
+    hipLaunchKernelGGL(quad, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
+  } else if (xcd) {
     const int64_t groups = std::max<int64_t>(splits_cap, 1) * (a.hkv / kWaves);
     const int64_t grid = static_cast<int64_t>(kXcds) * a.n_rows * ((groups + kXcds - 1) / kXcds) + a.pg_workers;
     if (grid > 0x7fffffff) return fail(RLT_EUNSUPPORTED, "rlt_paged_decode: too many work items");
