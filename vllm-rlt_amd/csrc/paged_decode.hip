@@ -89,19 +89,23 @@ constexpr int kMaxGrid = RLT_DECODE_MAX_GRID;
 #ifndef RLT_DECODE_XCD_SCHEDULE
 #define RLT_DECODE_XCD_SCHEDULE 1
 #endif
-// Launches of at most this many (row, kv head, split) items, splits counted
-// from the table width, give an item four waves: 2 waves per SIMD hold 2048
-// one-wave items at once, and below half of that the launch takes as long as
-// one item does.  Measured (16 heads, us, one wave against four): 4 rows of
-// 128-256 tokens 11.7 / 6.3, 1 of 256-512 13.9 / 9.3, 8 of 512-1024 18.0 /
-// 16.8 (640 items), 16 of 256-512 18.7 / 16.8 (768); 8 of 1024-2048 21.9 /
-// 25.5 (1152).  One-split launches of more than half as many only when the
-// table spans more than two quarters: 64 rows of 128-256 tokens 28.9 / 21.5,
-// of 32-64 11.4 / 13.3.
+// Launches that give an item four waves: of at most kQuadItems (row, kv head,
+// split) items, splits counted from the table width, kQuadRows when every row
+// is one split.  2 waves per SIMD hold 2048 one-wave items at once, and far
+// below that a launch takes as long as one item does.  Measured (16 heads, us,
+// one wave against four): 4 rows of 128-256 tokens 11.7 / 6.5, 1 of 256-512
+// 13.9 / 9.5, 8 of 512-1024 18.0 / 17.0 (512 items), 16 of 256-512 18.7 / 17.0
+// (512); 32 of 256-512 24.5 / 25.5, 16 of 512-1024 23.9 / 25.9 (1024).  One
+// split: 64 rows (1024 items) of 128-256 tokens 28.4 / 21.9, of 64-128 17.2 /
+// 16.7, of 32-64 11.3 / 13.6; rows of one quarter gain nothing (1 row of 32-64
+// 5.7 / 6.0).
 #ifndef RLT_DECODE_QUAD_ITEMS
-#define RLT_DECODE_QUAD_ITEMS 1024
+#define RLT_DECODE_QUAD_ITEMS 512
 #endif
 constexpr int kQuadItems = RLT_DECODE_QUAD_ITEMS;
+constexpr int kQuadRows = 2 * kQuadItems;
+// Rows of at most this many splits have their splits kept in quarters.
+constexpr int kQuarterSplits = 4;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, workgroups dispatched round-robin
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -434,10 +438,12 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   const int g = lane / LPT;
   const int s = lane % LPT;
   const uint32_t lane_dim = static_cast<uint32_t>(s * EPL);
-  // Items (quarters<T, D, G>) keep a quarter's softmax state and
-  // fold it into the split's at the quarter's end (fold below), in this order
-  // in every launch: so one wave that walks the quarters and four waves that
-  // take one each give the same bits, and the host may choose by the launch.
+  // Items of rows of up to kQuarterSplits splits (quarters<T, D, G>) keep a
+  // quarter's softmax state and fold it into the split's at the quarter's end
+  // (fold below), in this order in every launch: so one wave that walks the
+  // quarters and four waves that take one each give the same bits, and the host
+  // may choose by the launch.  The splits of longer rows are one piece: folding
+  // theirs cost large batches 0.3-0.8%, and few of them fill the chip.
   constexpr bool kQuarters = quarters<T, D, G>();
   static_assert(!QUAD || (kQuarters && XCD && !PREFIX), "shared items");
   constexpr int kStateFloats = G * (EPL + 2);
@@ -476,9 +482,12 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       store_new_token(r, h);
       return;
     }
-    const int quarter = split_len / kWaves;
-    const int t_begin = sp * split_len + (QUAD ? wave * quarter : 0);
-    const int t_end = min(len, t_begin + (QUAD ? quarter : split_len));
+    const bool quartered = kQuarters && ns <= kQuarterSplits;
+    if (QUAD && !quartered && wave != 0) return;
+    const bool shared = QUAD && quartered;  // by the workgroup's four waves
+    const int quarter = quartered ? split_len / kWaves : split_len;
+    const int t_begin = sp * split_len + (shared ? wave * quarter : 0);
+    const int t_end = min(len, t_begin + (shared ? quarter : split_len));
     const int last = t_end - 1;
     // Fused append: the row's write slot, read up front when this is its last split.
     int64_t wb = -1, wo = -1;
@@ -539,7 +548,8 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     };
     // One wave walking all quarters: after the tile that ends one.
     auto end_tile = [&](int t0) {
-      if constexpr (kQuarters && !QUAD) {
+      if constexpr (kQuarters) {
+        if (shared) return;
         if (((t0 + TILE - t_begin) & (quarter - 1)) == 0 || t0 + TILE >= t_end) {
           if (t0 - t_begin < quarter) {  // the first quarter: folding it into nothing is a copy
 #pragma unroll
@@ -621,7 +631,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       const int chunk_page = c0 / P;
       const int chunk_last = (c1 - 1) / P - chunk_page;  // <= 63
       int table_entry;
-      if (QUAD && early) table_entry = first_entry;  // a quarter is one chunk then
+      if (shared && early) table_entry = first_entry;  // a quarter is one chunk then
       else table_entry = lane <= chunk_last ? trow[chunk_page + lane] : 0;
       auto tile_pages = [&](int t0, int64_t (&blk)[PPT]) {
         const int rel0 = (t0 - c0) / P;
@@ -676,7 +686,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       u32x4 kp[NI], vp[NI];
       int64_t blk[PPT];
       if constexpr (QUAD) {
-        if (quarter == 2 * TILE) {
+        if (shared && quarter == 2 * TILE) {
           // Both tiles of a 64-token quarter in flight at once.  A second tile
           // past the end re-reads the last token and adds exactly nothing.
           u32x4 kp2[NI], vp2[NI];
@@ -748,7 +758,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       accumulate(vp, t0, sc);
       end_tile(t0);
     }
-    if constexpr (QUAD) {
+    if (shared) {
       // Wave 0 folds the quarters in order; the others hand theirs over.
       float* const mine = quarter_state + (wave - 1) * kStateFloats * 64 + lane;
       if (wave > 0) {
@@ -1683,7 +1693,8 @@ int launch_decode(DecodeArgs a, int64_t max_table_width, hipStream_t stream) {
   }
   const int64_t splits_cap = std::min<int64_t>(kMaxSplits, (max_tokens + kSplitTokens - 1) / kSplitTokens);
   const int64_t items_bound = static_cast<int64_t>(a.n_rows) * a.hkv * std::max<int64_t>(splits_cap, 1);
-  const bool few = items_bound <= (single_split && max_tokens <= kSplitTokens / 2 ? kQuadItems / 2 : kQuadItems);
+  const bool few = single_split ? max_tokens > 80 && items_bound <= (max_tokens > 128 ? kQuadRows : kQuadItems)
+                                : splits_cap <= kQuarterSplits && items_bound <= kQuadItems;
   const DecodeKernel quad = xcd && !prefix && few ? pick_quad<T>(a.d, G, append, single_split) : nullptr;
   if (quad) {
     const int64_t groups = std::max<int64_t>(splits_cap, 1) * a.hkv;
