@@ -1,4 +1,5 @@
-"""Compile the gfx950 HIP sources into the in-tree C-ABI library librlt_kv.so.
+"""Compile the gfx950 HIP sources into the in-tree C-ABI library librlt_kv.so,
+and the host calls (host_calls.cpp) into the extension module beside it.
 
 Every call recompiles (no up-to-date check): the caller decides when to build.
 """
@@ -8,6 +9,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -18,6 +20,7 @@ CSRC_DIR = PROJECT_DIR / "csrc"
 INCLUDE_DIR = REPO_DIR / "include"
 BUILD_DIR = PROJECT_DIR / "_build"
 LIBRARY = PACKAGE_DIR / "librlt_kv.so"
+HOST_CALLS = PACKAGE_DIR / "_host_calls.so"
 ARCH = "gfx950"
 
 # Packed-fp32 VALU forms are disabled for all device code; -O3 would otherwise
@@ -55,15 +58,35 @@ def _compile(source: Path) -> Path:
     return obj
 
 
+def build_host_calls() -> Path:
+    """The Python extension of csrc/host_calls.cpp, against the installed torch."""
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [INCLUDE_DIR, sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
+    tmp = HOST_CALLS.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall"]
+    cmd += [f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{i}" for i in includes)]
+    cmd += [str(CSRC_DIR / "host_calls.cpp"), f"-L{Path(torch.__file__).parent / 'lib'}"]
+    cmd += ["-ltorch_python", "-ltorch_cpu", "-lc10", "-o", str(tmp)]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"g++ failed on host_calls.cpp:\n{result.stderr}")
+    os.replace(tmp, HOST_CALLS)
+    return HOST_CALLS
+
+
 def build(jobs: int | None = None) -> Path:
-    """Compile every csrc/*.hip for gfx950 and link librlt_kv.so in the package."""
+    """Compile every csrc/*.hip for gfx950 and link librlt_kv.so in the package, beside its host calls."""
     BUILD_DIR.mkdir(parents=True, exist_ok=True)
     srcs = sources()
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC_DIR}")
     jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 2) // 2), 8)
     with ThreadPoolExecutor(jobs) as pool:
+        host_calls = pool.submit(build_host_calls)
         objects = list(pool.map(_compile, srcs))
+        host_calls.result()
     tmp = LIBRARY.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)]
     result = subprocess.run(cmd, capture_output=True, text=True)

@@ -142,11 +142,25 @@ SIGNATURES = {
 }
 
 _lib = None
+# The extension module of csrc/host_calls.cpp, bound to the loaded library:
+# the hot calls from tensors to the C ABI without ctypes (None before load()).
+host = None
+
+
+# Entry points host_calls.cpp calls, in bind()'s order.
+HOST_CALLED = (
+    "rlt_paged_decode",
+    "rlt_paged_decode_append",
+    "rlt_paged_decode_workspace_bytes",
+    "rlt_paged_prefill_split",
+    "rlt_paged_prefill_split_workspace_bytes",
+    "rlt_rope_kv_append",
+)
 
 
 def load(path: Path | str = LIBRARY_PATH) -> ctypes.CDLL:
     """Load (once) and type the library; raises if it has not been built."""
-    global _lib
+    global _lib, host
     if _lib is not None:
         return _lib
     path = Path(path)
@@ -160,6 +174,15 @@ def load(path: Path | str = LIBRARY_PATH) -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = restype
         fn.argtypes = argtypes
+    try:
+        from . import _host_calls
+    except ImportError as error:
+        raise RuntimeError(
+            f"the host calls beside {path.name} are missing: build the package first (python __graft_entry__.py build "
+            "or python -m vllm_rlt_amd._build)"
+        ) from error
+    _host_calls.bind(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in HOST_CALLED))
+    host = _host_calls
     _lib = lib
     return lib
 

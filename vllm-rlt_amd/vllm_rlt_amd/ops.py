@@ -28,6 +28,25 @@ def _require_rocm(*tensors: torch.Tensor) -> torch.device:
     return device
 
 
+def _host_calls(t: torch.Tensor):
+    """(module, current stream) of the direct host calls for the device tensor t, (None, 0) otherwise.
+
+    Their result is a tensor, a status of the library (_finish raises it), or
+    None for a call they leave to the checks and errors here.
+    """
+    if not t.is_cuda:
+        return None, 0
+    if _native.host is None:
+        _native.load()
+    return _native.host, stream_handle(t.device)
+
+
+def _finish(result, name: str) -> torch.Tensor:
+    if type(result) is int:
+        check(result, name)
+    return result
+
+
 def _require_int(t: torch.Tensor, dtype: torch.dtype, name: str, ndim: int = 1) -> None:
     if t.dtype != dtype or t.ndim != ndim:
         raise ValueError(f"{name} must be a {ndim}-D {dtype} tensor")
@@ -113,6 +132,13 @@ def rope_kv_append(
     (default: all of write_blocks) are written; q is rotated for every row.
     `out` may be q itself.
     """
+    host, stream = _host_calls(q)
+    if host is not None:
+        result = host.rope(
+            key_cache, value_cache, layer, write_blocks, write_offsets, q, k, v, cos, sin, out, n_rows, stream
+        )
+        if result is not None:
+            return _finish(result, "rlt_rope_kv_append")
     device = _require_rocm(key_cache, value_cache, write_blocks, write_offsets, q, k, v, cos, sin)
     if key_cache.shape != value_cache.shape or key_cache.stride() != value_cache.stride():
         raise ValueError("key_cache and value_cache must share shape and strides")
@@ -470,6 +496,15 @@ def paged_decode_append(
     groups' prefix pages are read once per launch
     (rlt_paged_decode_shared_prefix with its append arguments).
     """
+    if shared_prefix is None:
+        host, stream = _host_calls(q)
+        if host is not None:
+            result = host.decode(
+                q, key_cache, value_cache, block_tables, context_lengths, out, workspace, scale, stream, k_new, v_new,
+                write_blocks, write_offsets, n_write,
+            )
+            if result is not None:
+                return _finish(result, "rlt_paged_decode_append")
     device, rows, hq, hkv, d, page, nb, out = _decode_inputs(q, key_cache, value_cache, block_tables, context_lengths, out)
     _require_rocm(q, k_new, v_new, write_blocks, write_offsets)
     n = write_blocks.shape[0] if n_write is None else int(n_write)
@@ -521,6 +556,14 @@ def paged_decode(
     group's prefix pages are read once for all its rows
     (rlt_paged_decode_shared_prefix); the result is the same attention.
     """
+    if shared_prefix is None:
+        host, stream = _host_calls(q)
+        if host is not None:
+            result = host.decode(
+                q, key_cache, value_cache, block_tables, context_lengths, out, workspace, scale, stream
+            )
+            if result is not None:
+                return _finish(result, "rlt_paged_decode")
     device, rows, hq, hkv, d, page, nb, out = _decode_inputs(q, key_cache, value_cache, block_tables, context_lengths, out)
     if rows == 0:
         return out
@@ -597,6 +640,14 @@ def paged_prefill(
     workspace, long key ranges of short chunks are cut into segments whose
     partials are allocated here (rlt_paged_prefill_split).
     """
+    if workspace is None:
+        host, stream = _host_calls(q)
+        if host is not None:
+            result = host.prefill(
+                q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, stream
+            )
+            if result is not None:
+                return _finish(result, "rlt_paged_prefill")
     return _paged_prefill(
         q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace,
         workspace is None,

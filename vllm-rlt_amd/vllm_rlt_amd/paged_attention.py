@@ -106,9 +106,28 @@ class HipPagedAttention:
         """Grow the workspace for decode batches of up to `rows` rows."""
         return self.reserve(ops.decode_workspace_bytes(rows, num_q_heads, num_kv_heads, self.head_dim))
 
+    def _direct(self, q, key_cache, value_cache, block_tables, context_lengths, *append):
+        """The decode straight through the host calls when the workspace already holds it, else None."""
+        workspace = self._workspace
+        if workspace is None or not q.is_cuda:
+            return None
+        host, stream = ops._host_calls(q)
+        out = host.decode(
+            q, key_cache, value_cache, block_tables, context_lengths, None, workspace, None, stream, *append
+        )
+        if out is None:
+            return None
+        if torch._C._cuda_isCurrentStreamCapturing():
+            self._captured = True  # as reserve() notes it
+        return ops._finish(out, "rlt_paged_decode")
+
     def __call__(self, q, key_cache, value_cache, block_tables, context_lengths, shared_prefix=None):
         """Decode attention; `shared_prefix` (an ops.PrefixGroups, beyond the
         reference's signature) reads each group's aliased prefix pages once."""
+        if shared_prefix is None:
+            out = self._direct(q, key_cache, value_cache, block_tables, context_lengths)
+            if out is not None:
+                return out
         workspace = self.reserve_decode(q.shape[0], q.shape[1], key_cache.shape[2]) if q.shape[0] else None
         return ops.paged_decode(
             q, key_cache, value_cache, block_tables, context_lengths, workspace=workspace, shared_prefix=shared_prefix
@@ -121,6 +140,12 @@ class HipPagedAttention:
         The caller guarantees that no row reads a slot another row writes.
         `shared_prefix` as for __call__.
         """
+        if shared_prefix is None:
+            out = self._direct(
+                q, key_cache, value_cache, block_tables, context_lengths, k_new, v_new, write_blocks, write_offsets, n_write
+            )
+            if out is not None:
+                return out
         workspace = self.reserve_decode(q.shape[0], q.shape[1], key_cache.shape[2]) if q.shape[0] else None
         return ops.paged_decode_append(
             q, key_cache, value_cache, block_tables, context_lengths, k_new, v_new, write_blocks, write_offsets,
