@@ -125,3 +125,38 @@ def test_cut_key_ranges_beside_a_context_shorter_than_its_chunk():
     atol, rtol = TOL[torch.bfloat16]
     torch.testing.assert_close(out.cpu(), paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
     assert torch.count_nonzero(out.cpu()[row_lengths == 0]) == 0
+
+
+@pytest.mark.parametrize(
+    "hq,hkv,prefixes,chunks",
+    [
+        (16, 16, [0], [1]),
+        (16, 16, [31, 32, 33], [1, 31, 33]),  # rows and keys around a 32-row, 32-key tile
+        (8, 2, [255, 700], [65, 32]),  # every wave a tile; grouped heads
+        (3, 3, [9000], [40]),  # a wave's tiles past one batch of page ids
+        (4, 1, [0, 5] * 40, [0, 3] * 40),  # more sequences than lanes, empty ones among them
+    ],
+)
+def test_fp32_matrix_kernel(hq, hkv, prefixes, chunks):
+    q, kp, vp, tables, lens, cu, row_tables, row_lengths = ragged_prefill_case(
+        torch.float32, hq, hkv, 128, prefixes, chunks, 17
+    )
+    print(f"[prefill fp32] {hq}/{hkv} prefixes={prefixes[:3]} chunks={chunks[:3]}", flush=True)
+    atol, rtol = TOL[torch.float32]
+    for scale, sign in ((None, 1), (-(128**-0.5), -1)):
+        out = run_prefill(q, kp, vp, tables, lens, cu, chunks, scale=scale)
+        torch.testing.assert_close(out, paged_attention_cpu(sign * q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
+    # Rows off 16 bytes take the per-token path: the same attention.
+    shifted = torch.cat([q.new_zeros(1), q.flatten()]).cuda()[1:].view(q.shape)
+    apart = run_prefill(shifted, kp, vp, tables, lens, cu, chunks)
+    torch.testing.assert_close(apart, run_prefill(q, kp, vp, tables, lens, cu, chunks), atol=atol, rtol=rtol)
+
+
+def test_fp32_context_shorter_than_its_chunk():
+    chunks, contexts = [70, 3], [20, 1]
+    q, kp, vp, tables, _, cu, row_tables, _ = ragged_prefill_case(torch.float32, 4, 4, 128, [0, 0], chunks, 2)
+    row_lengths = torch.tensor([max(0, n - (c - 1 - i)) for n, c in zip(contexts, chunks) for i in range(c)], dtype=torch.int32)
+    out = run_prefill(q, kp, vp, tables, torch.tensor(contexts, dtype=torch.int32), cu, chunks)
+    atol, rtol = TOL[torch.float32]
+    torch.testing.assert_close(out, paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
+    assert torch.count_nonzero(out[row_lengths == 0]) == 0

@@ -34,6 +34,7 @@
 
 #include "common.hpp"
 #include "mfma.hpp"
+#include "prefill_f32.hpp"
 
 namespace rlt {
 namespace {
@@ -1143,14 +1144,14 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
     return fail(RLT_EINVAL, "rlt_paged_prefill: scale must be finite and nonzero");
 
   const int esize = dtype_size(dtype);
-  const bool mfma_ok = mfma_shape(head_dim, page_size, dtype) && q_strides[2] == 1 && out_strides[2] == 1 && kv_strides[3] == 1 &&
+  const bool rows_ok = q_strides[2] == 1 && out_strides[2] == 1 && kv_strides[3] == 1 &&
                        aligned16(q) && aligned16(out) && aligned16(key_cache) && aligned16(value_cache) &&
                        stride16(q_strides[0], esize) && stride16(q_strides[1], esize) &&
                        stride16(out_strides[0], esize) && stride16(out_strides[1], esize) &&
                        stride16(kv_strides[0], esize) && stride16(kv_strides[1], esize) &&
                        stride16(kv_strides[2], esize) && max_table_width > 0 && num_q_heads <= 4096 &&
                        kv_strides[1] >= 0 && kv_strides[1] * esize * page_size < (int64_t(1) << 31);
-  if (mfma_ok) {
+  if (rows_ok && mfma_shape(head_dim, page_size, dtype)) {
     PrefillArgs p{};
     p.q = q;
     p.q_row = q_strides[0];
@@ -1226,6 +1227,35 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
                 "requires 16-byte aligned q/out/cache rows and head_dim 64/128, page 16, bf16/fp16)",
                 (long long)workspace_bytes, (long long)need);
   if (!aligned16(workspace)) return fail(RLT_EINVAL, "rlt_paged_prefill: workspace must be 16-byte aligned");
+  if (rows_ok && dtype == RLT_FLOAT32 && head_dim == 128 && page_size == kPage) {
+    // The fp32 matrix-core kernel; the workspace stays unused (its size is
+    // the per-token path's, which rows off 16 bytes take).
+    PrefillF32Args p{};
+    p.q = static_cast<const float*>(q);
+    p.q_row = q_strides[0];
+    p.q_head = q_strides[1];
+    p.k = static_cast<const float*>(key_cache);
+    p.v = static_cast<const float*>(value_cache);
+    p.kv_block = kv_strides[0];
+    p.kv_token = kv_strides[1];
+    p.kv_head = kv_strides[2];
+    p.tables = block_tables;
+    p.table_stride = table_stride;
+    p.width = max_table_width;
+    p.lens = context_lengths;
+    p.cu = cu_seqlens_q;
+    p.out = static_cast<float*>(out);
+    p.o_row = out_strides[0];
+    p.o_head = out_strides[1];
+    p.num_seqs = static_cast<int>(num_seqs);
+    p.hq = static_cast<int>(num_q_heads);
+    p.hkv = static_cast<int>(num_kv_heads);
+    p.num_blocks = num_blocks;
+    p.total_q = static_cast<int>(total_q);
+    p.qscale = std::fabs(scale) * kLog2eP;
+    p.negate = scale < 0.f;
+    return launch_prefill_f32(p, as_stream(stream));
+  }
   const int64_t width = std::max<int64_t>(max_table_width, 1);
   char* ws = static_cast<char*>(workspace);
   ExpandArgs e{};

@@ -644,7 +644,8 @@ def paged_prefill(
         host, stream = _host_calls(q)
         if host is not None:
             result = host.prefill(
-                q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, stream
+                q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, stream,
+                None,
             )
             if result is not None:
                 return _finish(result, "rlt_paged_prefill")
