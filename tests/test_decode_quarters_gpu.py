@@ -2,7 +2,8 @@
 
 A split's tokens are kept in quarters; small launches give every quarter a
 wave, larger ones walk them with one.  Lengths sit at the edges of tiles (32),
-quarters (64) and splits (256).
+quarters (64) and splits (256).  Launches of few rows of two to four splits fold a
+row in one workgroup: the same bits again.
 """
 
 import pytest
@@ -67,6 +68,32 @@ def test_one_wave_and_four_give_the_same_bits(lengths, dtype, fused):
     atol, rtol = TOL[dtype]
     expect = paged_attention_cpu(case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
     torch.testing.assert_close(alone.cpu(), expect, atol=atol, rtol=rtol)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("splits,rows", [(2, 1), (2, 32), (3, 7), (3, 32), (4, 9), (4, 16)])
+def test_rows_in_one_workgroup_give_the_same_bits(splits, rows, dtype, fused):
+    edges = [n for n in LONGER if n <= 256 * splits] + [256 * splits - d for d in (1, 0, 64, 65, 33)]
+    lengths = [edges[(5 * i + splits) % len(edges)] for i in range(rows - 1)] + [256 * splits]
+    case = random_decode_case(lengths, hq=16, hkv=16, d=128, dtype=dtype, seed=rows + splits)
+    dev = case.to("cuda")
+    append = None
+    if fused:
+        last = (dev.lengths.long() - 1).clamp(min=0)
+        blocks = dev.tables[torch.arange(rows, device="cuda"), last // 16].long()
+        blocks[dev.lengths == 0] = -1
+        safe = blocks.clamp(min=0)
+        append = (dev.key_slice[safe, last % 16], dev.value_slice[safe, last % 16], blocks, last % 16)
+    few = launch(dev, slice(None), append)
+    copies = 1100 // rows  # past every limit of the small launches
+    many = random_case_copies(dev, copies)
+    batch = launch(many, slice(None), tuple(t.repeat((copies,) + (1,) * (t.ndim - 1)) for t in append) if append else None)
+    torch.cuda.synchronize()
+    assert torch.equal(batch, few.repeat(copies, 1, 1))
+    atol, rtol = TOL[dtype]
+    expect = paged_attention_cpu(case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
+    torch.testing.assert_close(few.cpu(), expect, atol=atol, rtol=rtol)
 
 
 def random_case_copies(case, copies):

@@ -93,9 +93,9 @@ constexpr int kMaxGrid = RLT_DECODE_MAX_GRID;
 // split) items, splits counted from the table width, kQuadRows when every row
 // is one split.  2 waves per SIMD hold 2048 one-wave items at once, and far
 // below that a launch takes as long as one item does.  Measured (16 heads, us,
-// one wave against four): 4 rows of 128-256 tokens 11.7 / 6.5, 1 of 256-512
-// 13.9 / 9.5, 8 of 512-1024 18.0 / 17.0 (512 items), 16 of 256-512 18.7 / 17.0
-// (512); 32 of 256-512 24.5 / 25.5, 16 of 512-1024 23.9 / 25.9 (1024).  One
+// one wave against four): 4 rows of 128-256 tokens 11.7 / 6.5, 1 of 512-1024
+// 13.7 / 9.6, 8 of 512-1024 18.0 / 17.2 (512 items; other rows of two to four
+// splits go to paged_decode_row_kernel, below).  One
 // split: 64 rows (1024 items) of 128-256 tokens 28.4 / 21.9, of 64-128 17.2 /
 // 16.7, of 32-64 11.3 / 13.6; rows of one quarter gain nothing (1 row of 32-64
 // 5.7 / 6.0).
@@ -106,6 +106,23 @@ constexpr int kQuadItems = RLT_DECODE_QUAD_ITEMS;
 constexpr int kQuadRows = 2 * kQuadItems;
 // Rows of at most this many splits have their splits kept in quarters.
 constexpr int kQuarterSplits = 4;
+// Launches that give a row's head one workgroup of eight waves, which fold its
+// splits themselves: no partials in memory and no merge kernel (4 us).  Up to
+// three splits: at most kRowItems (row, kv head) items, one workgroup a CU in
+// two rounds.  Four splits take two rounds of quarters (8 waves, 16 quarters)
+// on one CU, which pays only when the other CUs have rows of their own: from
+// past kRowFourMin (half the CUs) to kRowFourMax (all of them).  Measured (16 heads, us,
+// splits and merge against rows): 1 row of 256-512 tokens 9.5 / 7.4, 16 of
+// 256-512 17.1 / 12.8, 16 of 384-768 20.5 / 16.6, 32 of 256-512 (512 items)
+// 24.7 / 22.4, of 384-768 37.1 / 32.1; 64 of 256-512 (1024) 42.5 / 48.6.  Four
+// splits: 1 row of 512-1024 9.6 / 10.9, 8 (128 items) 17.2 / 16.3 warm but 17.9
+// / 18.0 with the pages in HBM, 16 (256) 24.4 / 21.4, 32 (512) 42.8 / 46.2.
+constexpr int kRowThreads = 512;
+#ifndef RLT_DECODE_ROW_ITEMS
+#define RLT_DECODE_ROW_ITEMS 512
+#endif
+constexpr int kRowItems = RLT_DECODE_ROW_ITEMS;
+constexpr int kRowFourMin = kRowItems / 4, kRowFourMax = kRowItems / 2;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, workgroups dispatched round-robin
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -419,9 +436,11 @@ __device__ __forceinline__ void shared_prefix_item(const DecodeArgs& a, int item
 // item stores the row's new token itself (APPEND), after its own reads, and no
 // merge kernel runs.
 // QUAD: the workgroup's four waves share one item, a quarter of its tokens
-// each (see kQuarters).
+// each (see kQuarters).  ROW: the workgroup's eight waves share all items of one
+// (row, kv head) of up to kQuarterSplits splits, and merge them: no partials,
+// no merge kernel.
 template <typename T, int D, int G, int P, int TILE, bool XCD, bool PREFIX, bool APPEND, bool ONE_SPLIT = false,
-          bool QUAD = false>
+          bool QUAD = false, bool ROW = false>
 __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const int blocks) {
   using PK = Packet<T>;
   constexpr int EPL = PK::N;      // elements of one token a lane owns
@@ -445,15 +464,77 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   // may choose by the launch.  The splits of longer rows are one piece: folding
   // theirs cost large batches 0.3-0.8%, and few of them fill the chip.
   constexpr bool kQuarters = quarters<T, D, G>();
-  static_assert(!QUAD || (kQuarters && XCD && !PREFIX), "shared items");
+  static_assert(!(QUAD || ROW) || (kQuarters && XCD && !PREFIX), "shared items");
   constexpr int kStateFloats = G * (EPL + 2);
-  __shared__ float quarter_state[QUAD ? (kWaves - 1) * kStateFloats * 64 : 1];
+  constexpr int kRowQuarters = kQuarterSplits * kWaves;
+  __shared__ float quarter_state[ROW ? kRowQuarters * kStateFloats * 64 : QUAD ? (kWaves - 1) * kStateFloats * 64 : 1];
+  // A quarter's state in LDS: value-major, a float per lane.
+  auto put_state = [&](int at, const float (&qm)[G], const float (&ql)[G], const float (&qa)[G][EPL]) {
+    float* const q = quarter_state + at * kStateFloats * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      q[(j * (EPL + 2)) * 64] = qm[j];
+      q[(j * (EPL + 2) + 1) * 64] = ql[j];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) q[(j * (EPL + 2) + 2 + e) * 64] = qa[j][e];
+    }
+  };
+  auto get_state = [&](int at, float (&qm)[G], float (&ql)[G], float (&qa)[G][EPL]) {
+    const float* const q = quarter_state + at * kStateFloats * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      qm[j] = q[(j * (EPL + 2)) * 64];
+      ql[j] = q[(j * (EPL + 2) + 1) * 64];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) qa[j][e] = q[(j * (EPL + 2) + 2 + e) * 64];
+    }
+  };
+  // A quarter's (qm, ql, qa) folded into the split's state; written out with
+  // fmaf so that every kernel rounds alike.
+  auto fold_into = [&](float (&sm)[G], float (&sl)[G], float (&sa)[G][EPL], const float (&qm)[G], const float (&ql)[G],
+                       const float (&qa)[G][EPL]) {
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      const float mn = fmaxf(sm[j], qm[j]);
+      const float fs = sm[j] == -INFINITY ? 0.f : fast_exp2(sm[j] - mn);
+      const float fq = qm[j] == -INFINITY ? 0.f : fast_exp2(qm[j] - mn);
+      sl[j] = fmaf(sl[j], fs, ql[j] * fq);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) sa[j][e] = fmaf(sa[j][e], fs, qa[j][e] * fq);
+      sm[j] = mn;
+    }
+  };
+  // The token groups (lanes that share s) merged: every lane ends with the whole split's.
+  auto merge_token_groups = [&](float (&m)[G], float (&l)[G], float (&acc)[G][EPL]) {
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      const float M = strided_max<LPT>(m[j]);
+      const float f = (m[j] == -INFINITY) ? 0.f : fast_exp2(m[j] - M);
+      l[j] = strided_sum<LPT>(l[j] * f);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) acc[j][e] = strided_sum<LPT>(acc[j][e] * f);
+      m[j] = M;
+    }
+  };
+  // A one-split row's output.
+  auto write_row = [&](int r, int h, const float (&l)[G], const float (&acc)[G][EPL]) {
+    if (g != 0) return;
+    T* orow = static_cast<T*>(a.out) + r * a.o_row + static_cast<int64_t>(h) * G * a.o_head + lane_dim;
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      float o[EPL];
+      const float inv = 1.f / l[j];
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) o[e] = acc[j][e] * inv;
+      *reinterpret_cast<u32x4*>(orow + j * a.o_head) = PK::pack(o);
+    }
+  };
 
   // A one-split launch's append: row r's new token of kv head h into its
   // write slot (skipped when the slot is outside the pool), by the lanes of
   // one token, after the item has read its pages.
   auto store_new_token = [&](const int r, const int h) {
-    if constexpr (APPEND && ONE_SPLIT) {
+    if constexpr (APPEND && (ONE_SPLIT || ROW)) {
       if (r >= a.n_write || g != 0) return;
       const int64_t b = a.write_blocks[r], o = a.write_offsets[r];
       if (b < 0 || b >= a.num_blocks || o < 0 || o >= a.page) return;
@@ -467,10 +548,28 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     }
   };
 
+  // QUAD and ROW: what an item needs beside its length and page ids, loaded
+  // with them (G = 1), so that K and V wait for one memory round trip only.
+  struct ItemLoads {
+    u32x4 q;
+    int64_t wb, wo;  // the row's write slot (APPEND)
+  };
+  auto load_item = [&](const int r, const int h) -> ItemLoads {
+    ItemLoads pre{};
+    pre.q = *reinterpret_cast<const u32x4*>(static_cast<const T*>(a.q) + r * a.q_row +
+                                            static_cast<int64_t>(h) * a.q_head + lane_dim);
+    if constexpr (APPEND) {  // a.n_write >= 1
+      pre.wb = a.write_blocks[min(r, a.n_write - 1)];
+      pre.wo = a.write_offsets[min(r, a.n_write - 1)];
+    }
+    return pre;
+  };
   // One (row r, kv head h, split sp) item per wave (per workgroup: QUAD).
-  // first_entry: QUAD's page ids of this wave's first 64 pages when early.
+  // first_entry: QUAD's and ROW's page ids of this wave's first 64 pages when
+  // early; qi: ROW's quarter of the row, whose state it leaves in LDS.
   auto process = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns,
-                     const bool early = false, const int first_entry = 0) {
+                     const bool early = false, const int first_entry = 0, const int qi = 0,
+                     const ItemLoads& pre = {}) {
     if (len <= 0) {
       if (QUAD && wave != 0) return;
       if (g == 0) {
@@ -482,19 +581,20 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       store_new_token(r, h);
       return;
     }
-    const bool quartered = kQuarters && ns <= kQuarterSplits;
+    const bool quartered = ROW || (kQuarters && ns <= kQuarterSplits);
     if (QUAD && !quartered && wave != 0) return;
-    const bool shared = QUAD && quartered;  // by the workgroup's four waves
+    const bool shared = (QUAD || ROW) && quartered;  // by the workgroup's waves
     const int quarter = quartered ? split_len / kWaves : split_len;
-    const int t_begin = sp * split_len + (shared ? wave * quarter : 0);
+    const int t_begin = ROW ? qi * quarter : sp * split_len + (shared ? wave * quarter : 0);
+    if (ROW && t_begin >= len) return;
     const int t_end = min(len, t_begin + (shared ? quarter : split_len));
     const int last = t_end - 1;
     // Fused append: the row's write slot, read up front when this is its last split.
     int64_t wb = -1, wo = -1;
     if constexpr (APPEND) {
       if (t_end == len && r < a.n_write) {
-        wb = a.write_blocks[r];
-        wo = a.write_offsets[r];
+        wb = QUAD || ROW ? pre.wb : a.write_blocks[r];
+        wo = QUAD || ROW ? pre.wo : a.write_offsets[r];
       }
     }
 
@@ -504,7 +604,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       const T* qrow = static_cast<const T*>(a.q) + r * a.q_row + static_cast<int64_t>(h) * G * a.q_head + lane_dim;
 #pragma unroll
       for (int j = 0; j < G; ++j) {
-        const u32x4 p = *reinterpret_cast<const u32x4*>(qrow + j * a.q_head);
+        const u32x4 p = QUAD || ROW ? pre.q : *reinterpret_cast<const u32x4*>(qrow + j * a.q_head);
         PK::unpack(p, qv[j]);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) qv[j][e] *= a.qscale;
@@ -522,8 +622,6 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       }
     };
     reset();
-    // The split's state, and a quarter's (qm, ql, qa) folded into it; written
-    // out with fmaf so that every kernel rounds alike.
     float sm[G], sl[G], sa[G][EPL];
     if constexpr (kQuarters) {
 #pragma unroll
@@ -535,16 +633,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       }
     }
     auto fold = [&](const float (&qm)[G], const float (&ql)[G], const float (&qa)[G][EPL]) {
-#pragma unroll
-      for (int j = 0; j < G; ++j) {
-        const float mn = fmaxf(sm[j], qm[j]);
-        const float fs = sm[j] == -INFINITY ? 0.f : fast_exp2(sm[j] - mn);
-        const float fq = qm[j] == -INFINITY ? 0.f : fast_exp2(qm[j] - mn);
-        sl[j] = fmaf(sl[j], fs, ql[j] * fq);
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) sa[j][e] = fmaf(sa[j][e], fs, qa[j][e] * fq);
-        sm[j] = mn;
-      }
+      fold_into(sm, sl, sa, qm, ql, qa);
     };
     // One wave walking all quarters: after the tile that ends one.
     auto end_tile = [&](int t0) {
@@ -685,7 +774,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       }
       u32x4 kp[NI], vp[NI];
       int64_t blk[PPT];
-      if constexpr (QUAD) {
+      if constexpr (QUAD || ROW) {
         if (shared && quarter == 2 * TILE) {
           // Both tiles of a 64-token quarter in flight at once.  A second tile
           // past the end re-reads the last token and adds exactly nothing.
@@ -758,32 +847,22 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       accumulate(vp, t0, sc);
       end_tile(t0);
     }
-    if (shared) {
-      // Wave 0 folds the quarters in order; the others hand theirs over.
-      float* const mine = quarter_state + (wave - 1) * kStateFloats * 64 + lane;
-      if (wave > 0) {
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-          mine[(j * (EPL + 2)) * 64] = m[j];
-          mine[(j * (EPL + 2) + 1) * 64] = l[j];
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) mine[(j * (EPL + 2) + 2 + e) * 64] = acc[j][e];
-        }
-      }
-      __syncthreads();  // and every read of the item's pages is done
-      if (wave > 0) return;
-      fold(m, l, acc);
-#pragma unroll
-      for (int w = 0; w < kWaves - 1; ++w) {
-        const float* const q = quarter_state + w * kStateFloats * 64 + lane;
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-          m[j] = q[(j * (EPL + 2)) * 64];
-          l[j] = q[(j * (EPL + 2) + 1) * 64];
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) acc[j][e] = q[(j * (EPL + 2) + 2 + e) * 64];
-        }
+    if constexpr (ROW) {
+      put_state(qi, m, l, acc);
+      return;
+    }
+    if constexpr (QUAD) {
+      if (shared) {
+        // Wave 0 folds the quarters in order; the others hand theirs over.
+        if (wave > 0) put_state(wave - 1, m, l, acc);
+        __syncthreads();  // and every read of the item's pages is done
+        if (wave > 0) return;
         fold(m, l, acc);
+#pragma unroll
+        for (int w = 0; w < kWaves - 1; ++w) {
+          get_state(w, m, l, acc);
+          fold(m, l, acc);
+        }
       }
     }
     if constexpr (kQuarters) {
@@ -796,29 +875,10 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       }
     }
 
-    // Merge the token groups (lanes that share s).
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      const float M = strided_max<LPT>(m[j]);
-      const float f = (m[j] == -INFINITY) ? 0.f : fast_exp2(m[j] - M);
-      l[j] = strided_sum<LPT>(l[j] * f);
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) acc[j][e] = strided_sum<LPT>(acc[j][e] * f);
-      m[j] = M;
-    }
+    merge_token_groups(m, l, acc);
 
     if (ns == 1) {
-      if (g == 0) {
-        T* orow = static_cast<T*>(a.out) + r * a.o_row + static_cast<int64_t>(h) * G * a.o_head + lane_dim;
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-          float o[EPL];
-          const float inv = 1.f / l[j];
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) o[e] = acc[j][e] * inv;
-          *reinterpret_cast<u32x4*>(orow + j * a.o_head) = PK::pack(o);
-        }
-      }
+      write_row(r, h, l, acc);
       store_new_token(r, h);
     } else {
       const int64_t slot = (static_cast<int64_t>(r) * a.hkv + h) * kMaxSplits + sp;
@@ -1064,11 +1124,85 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       if (ns == 1) store_new_token(r, h);
     }
   };
+  if constexpr (ROW) {
+    static_assert(G == 1 && kQuarterSplits * kSplitTokens / kRowQuarters == 2 * TILE, "two tiles a quarter");
+    constexpr int kRowWaves = kRowThreads / 64, kRounds = kRowQuarters / kRowWaves;
+    __shared__ float part_acc[kQuarterSplits][D];
+    __shared__ float2 part_ml[kQuarterSplits];
+    const int r = block / a.hkv, h = block - r * a.hkv;
+    const int width = static_cast<int>(a.max_len / P);
+    // The row's length, its page ids, q and the write slot go out together.
+    // Rows fit kQuarterSplits splits, so none is longer.
+    int entry[kRounds];
+#pragma unroll
+    for (int i = 0; i < kRounds; ++i)
+      entry[i] = a.tables[r * a.table_stride + min((wave + kRowWaves * i) * (2 * TILE / P) + (lane & 3), width - 1)];
+    const ItemLoads pre = load_item(r, h);
+    const int len = uniform(row_length(a, r));
+    const int ns = len > 0 ? (len + kSplitTokens - 1) / kSplitTokens : 1;
+    if (len <= 0) {
+      if (wave == 0) process(r, h, 0, len, kSplitTokens, ns);  // the zero row
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < kRounds; ++i) process(r, h, 0, len, kSplitTokens, ns, true, entry[i], wave + kRowWaves * i, pre);
+    __syncthreads();  // every quarter is in LDS, every page has been read
+    if (wave == kRowWaves - 1) store_new_token(r, h);
+    float m[G], l[G], acc[G][EPL];
+    if (wave < ns) {
+      // Wave sp folds split sp's quarters in order.
+      float qm[G], ql[G], qa[G][EPL];
+      get_state(wave * kWaves, m, l, acc);
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) {
+        const int at = wave * kWaves + w;
+        if (at * 2 * TILE >= len) break;
+        get_state(at, qm, ql, qa);
+        fold_into(m, l, acc, qm, ql, qa);
+      }
+      merge_token_groups(m, l, acc);
+      if (ns == 1) {
+        write_row(r, h, l, acc);
+      } else {
+        if (g == 0) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) part_acc[wave][lane_dim + e] = acc[0][e];
+        }
+        if (lane == 0) part_ml[wave] = make_float2(m[0], l[0]);
+      }
+    }
+    if (ns == 1) return;
+    __syncthreads();
+    if (wave != 0) return;
+    // The splits merged as the merge kernel does (merge_partials), operation by operation.
+    using L = MergeLoads<D>;
+    const float2 ml = lane < ns ? part_ml[lane] : make_float2(-INFINITY, 0.f);
+    const float M = strided_max<1>(ml.x);
+    const float w = lane < ns ? fast_exp2(ml.x - M) : 0.f;
+    const float inv = 1.f / group_sum<64>(ml.y * w);
+    const int c = lane % L::CH, q = lane / L::CH;
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kQuarterSplits / L::SPI; ++i) {
+      const int u = i * L::SPI + q;
+      const float wu = __shfl(w, u, 64);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = fmaf(u < ns ? part_acc[u][4 * c + e] : 0.f, wu, o[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = strided_sum<L::CH>(o[e]);
+    if (q == 0) {
+      T* orow = static_cast<T*>(a.out) + r * a.o_row + static_cast<int64_t>(h) * a.o_head;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) store_elem(orow + (4 * c + e) * a.o_dim, o[e] * inv);
+    }
+    return;
+  }
   if constexpr (QUAD) {
     // One (row, split, head) per workgroup, laid out as the XCD-affine
-    // schedule below with heads in place of head blocks.  The row's length,
-    // its page ids, and (in process) q and the write slot go out together when
-    // the split length does not depend on the row's own.
+    // schedule below with heads in place of head blocks.  The row's length, q,
+    // the write slot and, when the split length does not depend on the row's
+    // own, its page ids go out together.
     const int t = block / kXcds;
     const int r = t % a.n_rows;
     const int round = t / a.n_rows;
@@ -1080,10 +1214,11 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     const int page0 = sp * (kSplitTokens / P) + wave * (kSplitTokens / P / kWaves);
     const int width = static_cast<int>(a.max_len / P);
     const int entry = early && width > 0 ? a.tables[r * a.table_stride + min(page0 + (lane & 3), width - 1)] : 0;
+    const ItemLoads pre = load_item(r, h);
     const int len = uniform(row_length(a, r));
     int split_len, ns;
     split_plan(len, &split_len, &ns);
-    if (sp < ns) process(r, h, sp, len, split_len, ns, early, entry);
+    if (sp < ns) process(r, h, sp, len, split_len, ns, early, entry, 0, pre);
     return;
   }
   auto run_item = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns) {
@@ -1136,6 +1271,10 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
 
 // Four waves to an item (quarters<T, D, G> only), for launches that leave most of
 // the chip idle.
+template <typename T, int D, int G, int P, int TILE, bool APPEND>
+__global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))) void paged_decode_row_kernel(DecodeArgs a) {
+  split_pass<T, D, G, P, TILE, true, false, APPEND, false, false, true>(a, blockIdx.x, gridDim.x);
+}
 template <typename T, int D, int G, int P, int TILE, bool APPEND, bool ONE_SPLIT>
 __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a) {
   split_pass<T, D, G, P, TILE, true, false, APPEND, ONE_SPLIT, true>(a, blockIdx.x, gridDim.x);
@@ -1566,6 +1705,16 @@ DecodeKernel pick_quad(int d, int G, bool append, bool one_split) {
   return nullptr;
 }
 
+// The kernel that gives a whole (row, kv head) eight waves, likewise.
+template <typename T>
+DecodeKernel pick_row(int d, int G, bool append) {
+  if constexpr (quarters<T, 128, 1>()) {
+    if (d == 128 && G == 1)
+      return append ? paged_decode_row_kernel<T, 128, 1, 16, kTile, true> : paged_decode_row_kernel<T, 128, 1, 16, kTile, false>;
+  }
+  return nullptr;
+}
+
 // The fused-append split pass is compiled for the XCD-affine schedule (with
 // and without the shared-prefix check); other cases append first, then decode.
 template <typename T, int D, bool PREFIX>
@@ -1693,6 +1842,18 @@ int launch_decode(DecodeArgs a, int64_t max_table_width, hipStream_t stream) {
   }
   const int64_t splits_cap = std::min<int64_t>(kMaxSplits, (max_tokens + kSplitTokens - 1) / kSplitTokens);
   const int64_t items_bound = static_cast<int64_t>(a.n_rows) * a.hkv * std::max<int64_t>(splits_cap, 1);
+  // Rows of up to kQuarterSplits splits in launches of few of them: one
+  // workgroup a (row, kv head), no partials and no merge kernel.
+  const int64_t row_items = static_cast<int64_t>(a.n_rows) * a.hkv;
+  const bool whole_rows =
+      !single_split && (splits_cap < kQuarterSplits
+                            ? row_items <= kRowItems
+                            : splits_cap == kQuarterSplits && row_items > kRowFourMin && row_items <= kRowFourMax);
+  const DecodeKernel row = xcd && !prefix && whole_rows ? pick_row<T>(a.d, G, append) : nullptr;
+  if (row) {
+    hipLaunchKernelGGL(row, dim3(static_cast<unsigned>(row_items)), dim3(kRowThreads), 0, stream, a);
+    return check_launch("rlt_paged_decode(rows)");
+  }
   const bool few = single_split ? max_tokens > 80 && items_bound <= (max_tokens > 128 ? kQuadRows : kQuadItems)
                                 : splits_cap <= kQuarterSplits && items_bound <= kQuadItems;
   const DecodeKernel quad = xcd && !prefix && few ? pick_quad<T>(a.d, G, append, single_split) : nullptr;
