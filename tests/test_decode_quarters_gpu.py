@@ -96,6 +96,21 @@ def test_rows_in_one_workgroup_give_the_same_bits(splits, rows, dtype, fused):
     torch.testing.assert_close(few.cpu(), expect, atol=atol, rtol=rtol)
 
 
+@pytest.mark.parametrize("tokens", [16, 200, 256, 700, 1300])
+@pytest.mark.parametrize("heads", [(4, 4), (16, 16), (32, 8), (16, 4), (12, 12)])
+def test_every_row_and_head_is_served_once(heads, tokens):
+    """Left-over groups dealt out by rows: 1 to 7 of them (kv heads / 4 x splits, modulo 8), odd row counts."""
+    hq, hkv = heads
+    lengths = [1 + (37 * i) % tokens for i in range(66)] + [tokens]
+    case = random_decode_case(lengths, hq=hq, hkv=hkv, d=128, dtype=torch.bfloat16, seed=tokens)
+    dev = case.to("cuda")
+    out = launch(random_case_copies(dev, 5), slice(None), None).view(5, len(lengths), hq, 128)
+    assert all(torch.equal(out[0], o) for o in out[1:])
+    atol, rtol = TOL[torch.bfloat16]
+    expect = paged_attention_cpu(case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
+    torch.testing.assert_close(out[0].cpu(), expect, atol=atol, rtol=rtol)
+
+
 def random_case_copies(case, copies):
     """The case with its rows repeated; the copies read the same pages."""
     from dataclasses import replace

@@ -90,20 +90,19 @@ constexpr int kMaxGrid = RLT_DECODE_MAX_GRID;
 #define RLT_DECODE_XCD_SCHEDULE 1
 #endif
 // Launches that give an item four waves: of at most kQuadItems (row, kv head,
-// split) items, splits counted from the table width, kQuadRows when every row
-// is one split.  2 waves per SIMD hold 2048 one-wave items at once, and far
-// below that a launch takes as long as one item does.  Measured (16 heads, us,
-// one wave against four): 4 rows of 128-256 tokens 11.7 / 6.5, 1 of 512-1024
-// 13.7 / 9.6, 8 of 512-1024 18.0 / 17.2 (512 items; other rows of two to four
-// splits go to paged_decode_row_kernel, below).  One
-// split: 64 rows (1024 items) of 128-256 tokens 28.4 / 21.9, of 64-128 17.2 /
-// 16.7, of 32-64 11.3 / 13.6; rows of one quarter gain nothing (1 row of 32-64
-// 5.7 / 6.0).
+// split) items, splits counted from the table width, kQuadRows (one workgroup a
+// CU) when every row is one split.  2 waves per SIMD hold 2048 one-wave items at
+// once, and far below that a launch takes as long as one item does.  Measured
+// (16 heads, us, one wave against four): 1 row of 512-1024 tokens 13.7 / 9.6, 8
+// of 512-1024 18.0 / 17.2 (512 items; other rows of two to four splits go to
+// paged_decode_row_kernel, below).  One split: 4 rows of 128-256 tokens 11.7 /
+// 6.5, but 32 (512 items) of 128-256 15.4 / 17.1, of 64-128 9.6 / 14.6, 64 of
+// 128-256 21.1 / 30.0; rows of one quarter gain nothing (1 of 32-64 5.7 / 6.0).
 #ifndef RLT_DECODE_QUAD_ITEMS
 #define RLT_DECODE_QUAD_ITEMS 512
 #endif
 constexpr int kQuadItems = RLT_DECODE_QUAD_ITEMS;
-constexpr int kQuadRows = 2 * kQuadItems;
+constexpr int kQuadRows = kQuadItems / 2;
 // Rows of at most this many splits have their splits kept in quarters.
 constexpr int kQuarterSplits = 4;
 // Launches that give a row's head one workgroup of eight waves, which fold its
@@ -338,6 +337,41 @@ __device__ __forceinline__ int find_row(const int* prefix, int n, int x) {
 // slot lies inside the workspace) and the slots past ns are selected away
 // afterwards, so none of these loads waits for the row's length: the merge
 // costs one round trip to memory for the common split counts.
+// The XCD-affine schedule.  Workgroup b runs on XCD b % kXcds (the dispatcher's
+// round-robin; b counts from the first split-pass workgroup, after a whole
+// number of rounds of prefix workers).  Groups gi = split * head_blocks + block
+// are dealt out in rounds of kXcds, one to an XCD with all rows of it back to
+// back, so rows that alias the same pages in the same split read them together
+// from one L2.  Every second round runs in reverse: later splits have fewer
+// rows, and so each pair of rounds gives every XCD about the same number of
+// items.  The groups left over, fewer than kXcds, are dealt out by rows as well,
+// so that no XCD is left without work.  Measured, us, graph-timed, against
+// rounds rotated by one XCD and left-over groups whole on an XCD each: 16 kv heads,
+// rows of one split (4 groups: half the XCDs) 256 rows of 128-256 tokens 93.0 /
+// 68.5, 128 of 64-128 30.0 / 21.2, 161 of 595-724 165 / 147, 40 of 1-1300 50.4 /
+// 46.8, 64 of 512-4096 191.5 / 191.3; 8 kv heads 256 of 64-128 64.8 / 24.3, of
+// 300-512 140 / 108, 24 of 512-4096 61.3 / 57.8, 64 of 512-4096 130.0 / 126.3.
+// r and gi are named uniform: without, the grouped-query kernel spilled.
+// False: nothing for this workgroup.
+__device__ __forceinline__ bool xcd_item(const DecodeArgs& a, int b, int* r, int* gi) {
+  const int x = b % kXcds, t = b / kXcds;
+  const int rounds = a.xcd_groups / kXcds, rest = a.xcd_groups % kXcds;
+  // Whole rounds: row-major within a round.  Left over: row by row over the XCDs.
+  const int round = min(uniform(t / a.n_rows), rounds);
+  const bool whole = round < rounds;
+  const int i = t - round * a.n_rows;
+  const int left = i * kXcds + x;
+  const int row = uniform(left / max(rest, 1));
+  *r = whole ? i : row;
+  *gi = kXcds * round + (whole ? (round & 1 ? kXcds - 1 - x : x) : left - row * rest);
+  return *r < a.n_rows;
+}
+
+// Workgroups of the schedule above.
+int64_t xcd_grid(int64_t groups, int64_t n_rows) {
+  return groups / kXcds * kXcds * n_rows + (groups % kXcds * n_rows + kXcds - 1) / kXcds * kXcds;
+}
+
 template <int D>
 struct MergeLoads {
   static constexpr int CH = D / 4;     // 16-byte chunks of one split's accumulators
@@ -1203,11 +1237,8 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     // schedule below with heads in place of head blocks.  The row's length, q,
     // the write slot and, when the split length does not depend on the row's
     // own, its page ids go out together.
-    const int t = block / kXcds;
-    const int r = t % a.n_rows;
-    const int round = t / a.n_rows;
-    const int gi = kXcds * round + (block % kXcds + kXcds - round % kXcds) % kXcds;
-    if (gi >= a.xcd_groups) return;
+    int r, gi;
+    if (!xcd_item(a, block, &r, &gi)) return;
     const int sp = gi / a.hkv;
     const int h = gi - sp * a.hkv;
     const bool early = a.max_len <= kMaxSplits * kSplitTokens;
@@ -1227,22 +1258,10 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   };
 
   if constexpr (XCD) {
-    // XCD-affine schedule: workgroup b runs on XCD b % kXcds (the dispatcher's
-    // round-robin; b counts from the first split-pass workgroup, after a whole
-    // number of rounds of prefix workers) and owns one (row, split, block of
-    // kWaves heads).  Groups
-    // gi = split * head_blocks + block are dealt out in rounds of kXcds; in
-    // round k XCD x serves group k * kXcds + (x - k) mod kXcds, so every XCD
-    // takes early and late splits alike (later splits have fewer rows).  Each
-    // XCD walks its groups in order with all rows of a group back to back, so
-    // rows that alias the same pages in the same split read them together
-    // from one L2.  Items past a row's split count exit at once.
-    const int b = block;
-    const int t = b / kXcds;
-    const int r = t % a.n_rows;
-    const int round = t / a.n_rows;
-    const int gi = kXcds * round + (b % kXcds + kXcds - round % kXcds) % kXcds;
-    if (gi >= a.xcd_groups) return;
+    // XCD-affine schedule (xcd_item): a workgroup owns one (row, split, block
+    // of kWaves heads).  Items past a row's split count exit at once.
+    int r, gi;
+    if (!xcd_item(a, block, &r, &gi)) return;
     const int head_blocks = a.hkv / kWaves;
     const int sp = gi / head_blocks;
     const int h = (gi - sp * head_blocks) * kWaves + wave;
@@ -1854,17 +1873,17 @@ int launch_decode(DecodeArgs a, int64_t max_table_width, hipStream_t stream) {
     hipLaunchKernelGGL(row, dim3(static_cast<unsigned>(row_items)), dim3(kRowThreads), 0, stream, a);
     return check_launch("rlt_paged_decode(rows)");
   }
-  const bool few = single_split ? max_tokens > 80 && items_bound <= (max_tokens > 128 ? kQuadRows : kQuadItems)
+  const bool few = single_split ? max_tokens > 80 && items_bound <= kQuadRows
                                 : splits_cap <= kQuarterSplits && items_bound <= kQuadItems;
   const DecodeKernel quad = xcd && !prefix && few ? pick_quad<T>(a.d, G, append, single_split) : nullptr;
   if (quad) {
     const int64_t groups = std::max<int64_t>(splits_cap, 1) * a.hkv;
-    const int64_t grid = static_cast<int64_t>(kXcds) * a.n_rows * ((groups + kXcds - 1) / kXcds);
+    const int64_t grid = xcd_grid(groups, a.n_rows);
     a.xcd_groups = static_cast<int>(groups);
     hipLaunchKernelGGL(quad, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
   } else if (xcd) {
     const int64_t groups = std::max<int64_t>(splits_cap, 1) * (a.hkv / kWaves);
-    const int64_t grid = static_cast<int64_t>(kXcds) * a.n_rows * ((groups + kXcds - 1) / kXcds) + a.pg_workers;
+    const int64_t grid = xcd_grid(groups, a.n_rows) + a.pg_workers;
     if (grid > 0x7fffffff) return fail(RLT_EUNSUPPORTED, "rlt_paged_decode: too many work items");
     a.xcd_groups = static_cast<int>(groups);
     hipLaunchKernelGGL(tiled, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
