@@ -24,6 +24,10 @@
 // Workgroups are mapped XCD-major so one (head, sequence)'s query tiles share
 // an L2 while they stream the same prefix.
 //
+// Launches with few query tiles cut the keys into segments and merge them (see
+// kSegTiles).  fp32 rows of head_dim 128 on 16 bytes, page 16, have their own
+// kernel (paged_prefill_f32.hip).
+//
 // Other shapes expand each query row into a decode row (its own key length and
 // a copy of its sequence's table row) in the workspace and run the split-K
 // decode kernels -- the per-token causal rows the reference's non-FA4

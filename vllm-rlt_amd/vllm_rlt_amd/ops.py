@@ -633,9 +633,10 @@ def paged_prefill(
 ) -> torch.Tensor:
     """Packed bottom-right-causal prefill (FlashPagedAttention.prefill, flash_attention.py:66-96).
 
-    The MFMA path needs no workspace; other shapes (fp32, unaligned rows,
-    other head sizes) run each query row as a decode row and need
-    prefill_workspace_bytes(...) bytes, allocated here unless `workspace`
+    The 16-bit MFMA path needs no workspace.  Other shapes need
+    prefill_workspace_bytes(...) bytes: unaligned rows and other head or page
+    sizes run each query row as a decode row there (aligned fp32 rows of
+    head_dim 128, page 16 leave it unused).  They are allocated here unless `workspace`
     (a uint8 device tensor at least that large) is given.  Without a given
     workspace, long key ranges of short chunks are cut into segments whose
     partials are allocated here (rlt_paged_prefill_split).
