@@ -160,3 +160,27 @@ def test_fp32_context_shorter_than_its_chunk():
     atol, rtol = TOL[torch.float32]
     torch.testing.assert_close(out, paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
     assert torch.count_nonzero(out[row_lengths == 0]) == 0
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_fp32_value_that_is_not_finite_reaches_only_the_rows_that_see_it(bad):
+    # A masked key has P = 0, and 0 times its V is a NaN: rows before the token
+    # must be what they are without it, the rows that see it as the oracle has them.
+    prefixes, chunks = [70, 0, 300], [100, 40, 33]
+    q, kp, vp, tables, lens, cu, row_tables, row_lengths = ragged_prefill_case(
+        torch.float32, 8, 4, 128, prefixes, chunks, 23
+    )
+    clean = run_prefill(q, kp, vp, tables, lens, cu, chunks)
+    first = {}  # sequence -> its first poisoned token
+    for s, token, head, dims in ((0, 120, 1, slice(17, 18)), (0, 137, 3, slice(0, 128)), (1, 39, 2, slice(64, 70)),
+                                 (2, 317, 0, slice(127, 128))):
+        vp[int(tables[s, token // 16]), token % 16, head, dims] = bad
+        first.setdefault(s, token)
+    print(f"[prefill fp32] V {bad}", flush=True)
+    out = run_prefill(q, kp, vp, tables, lens, cu, chunks)
+    seq = torch.repeat_interleave(torch.arange(len(chunks)), torch.tensor(chunks))
+    before = row_lengths <= torch.tensor([first[int(s)] for s in seq])
+    assert before.any() and torch.equal(out[before], clean[before])
+    expect = paged_attention_cpu(q, kp, vp, row_tables, row_lengths)
+    atol, rtol = TOL[torch.float32]
+    torch.testing.assert_close(out, expect, atol=atol, rtol=rtol, equal_nan=True)

@@ -43,6 +43,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
   // q as S^T's B operand, then the waves' accumulators and (max, sum).
   __shared__ __align__(16) f32x4 lds[kWaves * 16 * 64];
   __shared__ float2 lds_ml[kWaves][64];
+  __shared__ int lds_odd;  // a masked tile's V holds elements that are not finite
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uniform(tid >> 6);
   const int half = lane >> 5, i = lane & 31;
@@ -85,8 +86,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
   const int keys = prefix + t0 + rows;           // keys of the tile's last row
   const int ntiles = keys > 0 ? (keys + kKeys - 1) / kKeys : 0;
   const int last = len - 1;
+  const int open = prefix + t0;                  // last key that every row of the tile sees
   const int kvh = h / (a.hq / a.hkv);
 
+  if (tid == 0) lds_odd = 0;
   // q rows into LDS, laid out as the lanes read them.
   for (int u = tid; u < kSteps * 64; u += 64 * kWaves) {
     const int s = u >> 6, l = u & 63;
@@ -147,6 +150,23 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     }
   };
 
+  // Tiles with keys that some row does not see.  P = 0 keeps a masked key's V
+  // out of a row only while it is finite, so what is not leaves the products
+  // here, and the store adds it to the rows that see it.
+  auto confine = [&](int n) __attribute__((always_inline)) {
+    if (kKeys * (wave + kWaves * n) + kKeys - 1 <= open) return;
+    bool odd = false;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool finite = (__float_as_uint(vr[u][e]) & 0x7f800000u) != 0x7f800000u;
+        odd |= !finite;
+        vr[u][e] = finite ? vr[u][e] : 0.f;
+      }
+    if (odd) lds_odd = 1;
+  };
+
   const int mine = ntiles > wave ? (ntiles - wave + kWaves - 1) / kWaves : 0;
   if (mine > 0) {
     load_ids(0);
@@ -203,6 +223,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[c][r] *= corr;
+    confine(n);
 #pragma unroll
     for (int r = 0; r < 8; ++r)
 #pragma unroll
@@ -213,6 +234,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
       load_k(n + 1);
     }
     __builtin_amdgcn_sched_barrier(0);
+    confine(n);
 #pragma unroll
     for (int r = 0; r < 8; ++r)
 #pragma unroll
@@ -239,6 +261,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
   }
   const float inv = total > 0.f ? 1.f / total : 0.f;  // a row that sees no key is written as zeros
   if (i >= rows) return;
+  const bool odd = uniform(lds_odd);
   float* const orow = a.out + (row0 + my_row) * a.o_row + static_cast<int64_t>(h) * a.o_head;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -252,7 +275,18 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] *= inv;
-    *reinterpret_cast<f32x4*>(orow + 4 * (8 * (r >> 2) + 4 * half + (r & 3))) = o;
+    const int dim = 4 * (8 * (r >> 2) + 4 * half + (r & 3));
+    if (odd) {
+      for (int key = max(open + 1, 0) / kKeys * kKeys; key <= limit; ++key) {
+        const int32_t b = trow[key / kPage];
+        const int64_t blk = (b < 0 || b >= a.num_blocks) ? 0 : b;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(vbase + blk * a.kv_block + key % kPage * a.kv_token + dim);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u) o[e] += v[e];
+      }
+    }
+    *reinterpret_cast<f32x4*>(orow + dim) = o;
   }
 }
 
