@@ -111,6 +111,26 @@ def test_every_row_and_head_is_served_once(heads, tokens):
     torch.testing.assert_close(out[0].cpu(), expect, atol=atol, rtol=rtol)
 
 
+@pytest.mark.parametrize("lengths", [[160, 200], [160, 420], [160, 1000], [160, 3000]], ids=str)
+def test_a_tile_of_minus_infinity_scores(lengths):
+    # The first tiles of a split, of a quarter and of a later split's quarter hold
+    # only scores of -inf: weights of 0, as the oracle has them.
+    case = random_decode_case(lengths, hq=16, hkv=16, d=128, dtype=torch.bfloat16, seed=lengths[1])
+    case.q[:, 3, 7] = 1.5
+    for r, n in enumerate(lengths):
+        for first in (0, 64, 320):
+            if first + 32 < n:
+                case.key_slice[case.tables[r, first // 16 : first // 16 + 2].long(), :, 3, 7] = float("-inf")
+    expect = paged_attention_cpu(case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
+    assert expect.isfinite().all()
+    dev = case.to("cuda")
+    atol, rtol = TOL[torch.bfloat16]
+    for copies in (1, 12, 200):  # four waves an item, whole rows, one wave an item
+        out = launch(random_case_copies(dev, copies), slice(None), None).view(copies, len(lengths), 16, 128)
+        assert all(torch.equal(out[0], o) for o in out[1:])
+        torch.testing.assert_close(out[0].cpu(), expect, atol=atol, rtol=rtol)
+
+
 def random_case_copies(case, copies):
     """The case with its rows repeated; the copies read the same pages."""
     from dataclasses import replace

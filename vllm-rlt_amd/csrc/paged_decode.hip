@@ -724,12 +724,13 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
 #pragma unroll
         for (int i = 1; i < NI; ++i) tmax = fmaxf(tmax, sc[j][i]);
         const float mn = fmaxf(m[j], tmax);
-        const float corr = (mn == -INFINITY) ? 1.f : fast_exp2(m[j] - mn);
+        const float mb = (mn == -INFINITY) ? 0.f : mn;  // scores of -inf only: P = 0, not exp2(-inf + inf)
+        const float corr = fast_exp2(m[j] - mb);
         float psum = 0.f;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
           const bool valid = t0 + i * TPI + g <= last;
-          p[j][i] = valid ? fast_exp2(sc[j][i] - mn) : 0.f;
+          p[j][i] = valid ? fast_exp2(sc[j][i] - mb) : 0.f;
           psum += p[j][i];
         }
         l[j] = l[j] * corr + psum;
