@@ -156,6 +156,7 @@ struct DecodeArgs {
   float2* ws_ml;  // [rows][hkv][kMaxSplits][G]  (max in log2 units, sum)
   int n_rows, hkv, hq, d, page;
   int xcd_groups;  // > 0: XCD-affine schedule over this many (split, head block) groups
+  uint32_t rows_inverse, rest_inverse;  // inverse() of n_rows and of xcd_groups % kXcds
   int64_t num_blocks;
   int64_t max_len;  // table width * page: lengths are clamped to what the table covers
   float qscale;     // softmax scale * log2(e)
@@ -325,18 +326,13 @@ __device__ __forceinline__ int find_row(const int* prefix, int n, int x) {
   return lo;
 }
 
-// Merges the split partials of (row r, kv head h, q head j) into the output
-// when the row has ns >= 2 splits.  Lane sp holds split sp's (max, sum)
-// (kMaxSplits == 64 == wave size), so the global max and the normaliser are
-// two wave reductions.  The accumulators are read 16 bytes per lane: lane
-// (q, c) of a load reads dims 4c .. 4c + 3 of split i * SPI + q, so one load
-// instruction covers SPI whole splits.  Each lane sums its splits in split
-// order, then the SPI lanes of one chunk are added by a fixed butterfly, so
-// the result depends only on the row's own partials.  The (max, sum) of all
-// 64 slots and the first batch of SPB splits are loaded whatever ns is (every
-// slot lies inside the workspace) and the slots past ns are selected away
-// afterwards, so none of these loads waits for the row's length: the merge
-// costs one round trip to memory for the common split counts.
+// x / n from inverse(n): the product is at most one short.
+uint32_t inverse(uint32_t n) { return n ? 0xffffffffu / n : 0; }
+__device__ __forceinline__ uint32_t divide(uint32_t x, uint32_t n, uint32_t inverse_n) {
+  const uint32_t q = __umulhi(x, inverse_n);
+  return x - q * n >= n ? q + 1 : q;
+}
+
 // The XCD-affine schedule.  Workgroup b runs on XCD b % kXcds (the dispatcher's
 // round-robin; b counts from the first split-pass workgroup, after a whole
 // number of rounds of prefix workers).  Groups gi = split * head_blocks + block
@@ -353,25 +349,48 @@ __device__ __forceinline__ int find_row(const int* prefix, int n, int x) {
 // 300-512 140 / 108, 24 of 512-4096 61.3 / 57.8, 64 of 512-4096 130.0 / 126.3.
 // r and gi are named uniform: without, the grouped-query kernel spilled.
 // False: nothing for this workgroup.
+// Every workgroup runs this before its first load, the many that exit at once
+// included, so the divisions are multiplications by what the host has divided.
 __device__ __forceinline__ bool xcd_item(const DecodeArgs& a, int b, int* r, int* gi) {
-  const int x = b % kXcds, t = b / kXcds;
-  const int rounds = a.xcd_groups / kXcds, rest = a.xcd_groups % kXcds;
+  const uint32_t x = b % kXcds, t = static_cast<uint32_t>(b) / kXcds;
+  const uint32_t rounds = a.xcd_groups / kXcds, rest = a.xcd_groups % kXcds;
   // Whole rounds: row-major within a round.  Left over: row by row over the XCDs.
-  const int round = min(uniform(t / a.n_rows), rounds);
-  const bool whole = round < rounds;
-  const int i = t - round * a.n_rows;
-  const int left = i * kXcds + x;
-  const int row = uniform(left / max(rest, 1));
-  *r = whole ? i : row;
-  *gi = kXcds * round + (whole ? (round & 1 ? kXcds - 1 - x : x) : left - row * rest);
-  return *r < a.n_rows;
+  const uint32_t round = min(divide(t, a.n_rows, a.rows_inverse), rounds);
+  const uint32_t i = t - round * a.n_rows;
+  if (round < rounds) {
+    *r = uniform(static_cast<int>(i));
+    *gi = uniform(static_cast<int>(kXcds * round + (round & 1 ? kXcds - 1 - x : x)));
+    return true;
+  }
+  if (rest == 0) return false;
+  const uint32_t left = i * kXcds + x;
+  const uint32_t row = divide(left, rest, a.rest_inverse);
+  *r = uniform(static_cast<int>(row));
+  *gi = uniform(static_cast<int>(kXcds * rounds + left - row * rest));
+  return row < static_cast<uint32_t>(a.n_rows);
 }
 
-// Workgroups of the schedule above.
-int64_t xcd_grid(int64_t groups, int64_t n_rows) {
+// Sets the schedule up and returns its workgroups.
+int64_t xcd_grid(DecodeArgs& a, int64_t groups) {
+  const int64_t n_rows = a.n_rows;
+  a.xcd_groups = static_cast<int>(groups);
+  a.rows_inverse = inverse(static_cast<uint32_t>(n_rows));
+  a.rest_inverse = inverse(static_cast<uint32_t>(groups % kXcds));
   return groups / kXcds * kXcds * n_rows + (groups % kXcds * n_rows + kXcds - 1) / kXcds * kXcds;
 }
 
+// Merges the split partials of (row r, kv head h, q head j) into the output
+// when the row has ns >= 2 splits.  Lane sp holds split sp's (max, sum)
+// (kMaxSplits == 64 == wave size), so the global max and the normaliser are
+// two wave reductions.  The accumulators are read 16 bytes per lane: lane
+// (q, c) of a load reads dims 4c .. 4c + 3 of split i * SPI + q, so one load
+// instruction covers SPI whole splits.  Each lane sums its splits in split
+// order, then the SPI lanes of one chunk are added by a fixed butterfly, so
+// the result depends only on the row's own partials.  The (max, sum) of all
+// 64 slots and the first batch of SPB splits are loaded whatever ns is (every
+// slot lies inside the workspace) and the slots past ns are selected away
+// afterwards, so none of these loads waits for the row's length: the merge
+// costs one round trip to memory for the common split counts.
 template <int D>
 struct MergeLoads {
   static constexpr int CH = D / 4;     // 16-byte chunks of one split's accumulators
@@ -1879,14 +1898,12 @@ int launch_decode(DecodeArgs a, int64_t max_table_width, hipStream_t stream) {
   const DecodeKernel quad = xcd && !prefix && few ? pick_quad<T>(a.d, G, append, single_split) : nullptr;
   if (quad) {
     const int64_t groups = std::max<int64_t>(splits_cap, 1) * a.hkv;
-    const int64_t grid = xcd_grid(groups, a.n_rows);
-    a.xcd_groups = static_cast<int>(groups);
+    const int64_t grid = xcd_grid(a, groups);
     hipLaunchKernelGGL(quad, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
   } else if (xcd) {
     const int64_t groups = std::max<int64_t>(splits_cap, 1) * (a.hkv / kWaves);
-    const int64_t grid = xcd_grid(groups, a.n_rows) + a.pg_workers;
+    const int64_t grid = xcd_grid(a, groups) + a.pg_workers;
     if (grid > 0x7fffffff) return fail(RLT_EUNSUPPORTED, "rlt_paged_decode: too many work items");
-    a.xcd_groups = static_cast<int>(groups);
     hipLaunchKernelGGL(tiled, dim3(static_cast<unsigned>(grid)), dim3(64 * kWaves), 0, stream, a);
   } else {
     const int64_t items = static_cast<int64_t>(a.n_rows) * a.hkv * std::max<int64_t>(splits_cap, 1);
