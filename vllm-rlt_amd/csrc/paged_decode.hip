@@ -1319,12 +1319,17 @@ __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a) {
   split_pass<T, D, G, P, TILE, true, false, APPEND, ONE_SPLIT, true>(a, blockIdx.x, gridDim.x);
 }
 
-// Items with quarters would fit three waves per SIMD (142 VGPRs), which streams
-// more slowly than two (64 rows of 512-4096 tokens 194.5 against 192.5 us, 256
-// of 1024-8192 1533 against 1527 us): naming v169 holds the kernel at two.
+// With quarters and an append the kernel would fit three waves per SIMD (136
+// VGPRs), which streams more slowly than two: 64 rows of 512-4096 tokens 194.2
+// against 190.7 us, 100 of 100-512 62.2 / 59.5.  Naming v169 holds it at two,
+// where it was before it had quarters (fp16 ran at four: 100 rows of 64-80 in
+// 4096-token tables 22.8 unnamed, 24.3 at two).  Without an append it runs at four (127
+// VGPRs): 64 rows of 512-4096 196.4 against 193.8 at two, but 40 of 512-1024
+// 51.8 / 56.1, and 100 of 1-64 in 4096-token tables, whose other splits'
+// workgroups only start and exit, 15.9 / 19.4.
 template <typename T, int D, int G, int P, int TILE, bool XCD, bool APPEND, bool ONE_SPLIT>
 __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
-  if constexpr (quarters<T, D, G>() && !ONE_SPLIT) asm volatile("" ::: "v169");
+  if constexpr (quarters<T, D, G>() && std::is_same_v<T, bf16> && APPEND && !ONE_SPLIT) asm volatile("" ::: "v169");
   split_pass<T, D, G, P, TILE, XCD, false, APPEND, ONE_SPLIT>(a, blockIdx.x, gridDim.x);
 }
 
