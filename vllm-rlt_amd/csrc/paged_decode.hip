@@ -514,9 +514,11 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   // quarter's softmax state and fold it into the split's at the quarter's end
   // (fold below), in this order in every launch: so one wave that walks the
   // quarters and four waves that take one each give the same bits, and the host
-  // may choose by the launch.  The splits of longer rows are one piece: folding
+  // may choose by the launch (of the XCD-affine schedule: the launches without it
+  // have no four-wave form, and folding cost them 2-3%).  The splits of longer
+  // rows are one piece: folding
   // theirs cost large batches 0.3-0.8%, and few of them fill the chip.
-  constexpr bool kQuarters = quarters<T, D, G>();
+  constexpr bool kQuarters = XCD && quarters<T, D, G>();
   static_assert(!(QUAD || ROW) || (kQuarters && XCD && !PREFIX), "shared items");
   constexpr int kStateFloats = G * (EPL + 2);
   constexpr int kRowQuarters = kQuarterSplits * kWaves;
