@@ -1321,6 +1321,13 @@ __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a) {
   split_pass<T, D, G, P, TILE, true, false, APPEND, ONE_SPLIT, true>(a, blockIdx.x, gridDim.x);
 }
 
+// fp32 with one q head per kv head: two waves per SIMD, which the append would
+// otherwise miss by a few registers.
+template <typename T, int D, int G>
+constexpr bool two_waves() {
+  return G == 1 && D == 128 && sizeof(T) == 4;
+}
+
 // With quarters and an append the kernel would fit three waves per SIMD (136
 // VGPRs), which streams more slowly than two: 64 rows of 512-4096 tokens 194.2
 // against 190.7 us, 100 of 100-512 62.2 / 59.5.  Naming v169 holds it at two,
@@ -1330,7 +1337,8 @@ __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a) {
 // 51.8 / 56.1, and 100 of 1-64 in 4096-token tables, whose other splits'
 // workgroups only start and exit, 15.9 / 19.4.
 template <typename T, int D, int G, int P, int TILE, bool XCD, bool APPEND, bool ONE_SPLIT>
-__global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(two_waves<T, D, G>() ? 2 : 1))) void
+paged_decode_kernel(DecodeArgs a) {
   if constexpr (quarters<T, D, G>() && std::is_same_v<T, bf16> && APPEND && !ONE_SPLIT) asm volatile("" ::: "v169");
   split_pass<T, D, G, P, TILE, XCD, false, APPEND, ONE_SPLIT>(a, blockIdx.x, gridDim.x);
 }
