@@ -131,6 +131,23 @@ def test_a_tile_of_minus_infinity_scores(lengths):
         torch.testing.assert_close(out[0].cpu(), expect, atol=atol, rtol=rtol)
 
 
+@pytest.mark.parametrize("lengths", [[32, 96, 224], [96, 288, 480], [96, 544, 992]], ids=str)
+def test_an_infinite_value_in_the_last_token(lengths):
+    # Rows that end with a full first tile of a quarter: its second tile is loaded
+    # beyond the row, from the last token, and 0 x Inf would be a NaN.
+    case = random_decode_case(lengths, hq=16, hkv=16, d=128, dtype=torch.bfloat16, seed=lengths[1])
+    for r, n in enumerate(lengths):
+        case.value_slice[int(case.tables[r, (n - 1) // 16]), (n - 1) % 16, 3, 7] = float("inf")
+    expect = paged_attention_cpu(case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
+    assert (expect == float("inf")).sum() == len(lengths) and not expect.isnan().any()
+    dev = case.to("cuda")
+    atol, rtol = TOL[torch.bfloat16]
+    for copies in (1, 8, 200):  # four waves an item, whole rows, one wave an item
+        out = launch(random_case_copies(dev, copies), slice(None), None).view(copies, len(lengths), 16, 128)
+        assert all(torch.equal(out[0], o) for o in out[1:])
+        torch.testing.assert_close(out[0].cpu(), expect, atol=atol, rtol=rtol)
+
+
 def random_case_copies(case, copies):
     """The case with its rows repeated; the copies read the same pages."""
     from dataclasses import replace

@@ -833,7 +833,8 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       if constexpr (QUAD || ROW) {
         if (shared && quarter == 2 * TILE) {
           // Both tiles of a 64-token quarter in flight at once.  A second tile
-          // past the end re-reads the last token and adds exactly nothing.
+          // past the end re-reads the last token, whose V need not be finite,
+          // and is not used.
           u32x4 kp2[NI], vp2[NI];
           int64_t blk2[PPT];
           tile_pages(c0, blk);
@@ -853,8 +854,10 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
           float sc[G][NI];
           scores(kp, c0, sc);
           accumulate(vp, c0, sc);
-          scores(kp2, c0 + TILE, sc);
-          accumulate(vp2, c0 + TILE, sc);
+          if (c0 + TILE < t_end) {
+            scores(kp2, c0 + TILE, sc);
+            accumulate(vp2, c0 + TILE, sc);
+          }
           continue;
         }
       }
