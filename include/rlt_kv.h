@@ -364,16 +364,20 @@ int rlt_paged_prefill(const void* q, const int64_t* q_strides, const void* key_c
                       void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
- * rlt_paged_prefill with room for key segments.  Same arguments, contract and
- * refusals.  On the MFMA path (head_dim 128), a launch of few query tiles over
- * long contexts has the sequences' keys cut into segments that run side by
- * side, each row's segment partials in `workspace`, merged by a second kernel.
- * Whether and how often depends on the launch's shapes (total_q, num_seqs,
- * max_table_width, num_q_heads) and each sequence's length, so a row's last
- * bits may depend on how many query rows share its launch; rlt_paged_prefill,
- * or a workspace below rlt_paged_prefill_split_workspace_bytes() (or NULL),
- * never cuts.  The workspace must not be shared by calls that overlap.  Off
- * the MFMA path the workspace is rlt_paged_prefill's, and its size the same.
+ * rlt_paged_prefill with the forms that depend on what shares the launch.  Same
+ * arguments, contract and refusals.  On the MFMA path (head_dim 128), a launch
+ * of few query tiles over long contexts has the sequences' keys cut into
+ * segments that run side by side, each row's segment partials in `workspace`,
+ * merged by a second kernel; a workspace below
+ * rlt_paged_prefill_split_workspace_bytes() (or NULL) never cuts.  fp32 rows
+ * (head_dim 128, page 16, 16-byte rows) of launches with enough of them run on
+ * the fp32 matrix instructions instead of the per-token path.  Both choices
+ * depend on the launch's shapes (total_q, num_seqs, max_seqlen_q,
+ * max_table_width and the heads) and each sequence's length, so a row's last
+ * bits may depend on how many query rows share its launch; rlt_paged_prefill's
+ * depend on the row's own sequence only.  The workspace must not be shared by
+ * calls that overlap.  Off the MFMA path the workspace is rlt_paged_prefill's,
+ * and its size the same.
  */
 int rlt_paged_prefill_split(const void* q, const int64_t* q_strides, const void* key_cache,
                             const void* value_cache, const int64_t* kv_strides,

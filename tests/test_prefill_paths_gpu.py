@@ -184,3 +184,55 @@ def test_fp32_value_that_is_not_finite_reaches_only_the_rows_that_see_it(bad):
     expect = paged_attention_cpu(q, kp, vp, row_tables, row_lengths)
     atol, rtol = TOL[torch.float32]
     torch.testing.assert_close(out, expect, atol=atol, rtol=rtol, equal_nan=True)
+
+
+@pytest.mark.parametrize(
+    "hq,hkv,prefixes,chunks",
+    [(16, 16, [4000], [1]), (16, 16, [2000, 700], [8, 3]), (32, 8, [2500], [7]), (8, 8, [0, 40, 900], [1, 1, 16])],
+)
+def test_few_fp32_rows_stay_on_the_per_token_path(hq, hkv, prefixes, chunks):
+    # A row tile of the matrix-core kernel costs 1 row as much as 32, and one
+    # workgroup walks all its keys: few rows are decoded one by one, as by paged_decode.
+    from vllm_rlt_amd import ops
+
+    q, kp, vp, tables, lens, cu, row_tables, row_lengths = ragged_prefill_case(
+        torch.float32, hq, hkv, 128, prefixes, chunks, 31
+    )
+    out = run_prefill(q, kp, vp, tables, lens, cu, chunks)
+    rows = ops.paged_decode(q.cuda(), kp.cuda(), vp.cuda(), row_tables.cuda(), row_lengths.int().cuda())
+    assert torch.equal(out, rows.cpu())
+    given = torch.empty(
+        ops.prefill_workspace_bytes(len(q), len(chunks), tables.shape[1], hq, hkv, 128, 16, torch.float32),
+        dtype=torch.uint8, device="cuda",
+    )
+    assert torch.equal(run_prefill(q, kp, vp, tables, lens, cu, chunks, workspace=given), out)
+    atol, rtol = TOL[torch.float32]
+    torch.testing.assert_close(out, paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
+
+
+@pytest.mark.parametrize(
+    "hq,hkv,prefixes,chunks",
+    [
+        (32, 1, [0], [1]),
+        (32, 1, [9000], [40]),  # a wave's tiles past one batch of page ids
+        (4, 1, [0, 205] * 40, [0, 40] * 40),  # more sequences than lanes, empty ones among them
+        (3, 3, [31, 32, 33], [255, 256, 257]),
+    ],
+)
+def test_fp32_matrix_kernel_where_it_is_taken(hq, hkv, prefixes, chunks):
+    from vllm_rlt_amd import ops
+
+    q, kp, vp, tables, lens, cu, row_tables, row_lengths = ragged_prefill_case(
+        torch.float32, hq, hkv, 128, prefixes, chunks, 37
+    )
+    print(f"[prefill fp32] {hq}/{hkv} prefixes={prefixes[:3]} chunks={chunks[:3]}", flush=True)
+    out = run_prefill(q, kp, vp, tables, lens, cu, chunks)
+    rows = ops.paged_decode(q.cuda(), kp.cuda(), vp.cuda(), row_tables.cuda(), row_lengths.int().cuda())
+    if len(q) > 1:
+        assert not torch.equal(out, rows.cpu())  # not the per-token path, whose bits are these
+    atol, rtol = TOL[torch.float32]
+    torch.testing.assert_close(out, paged_attention_cpu(q, kp, vp, row_tables, row_lengths), atol=atol, rtol=rtol)
+    short = [max(1, n // 3) for n in lens.tolist()]  # a context shorter than its chunk: rows that see no key
+    seen = torch.tensor([max(0, n - (c - 1 - i)) for n, c in zip(short, chunks) for i in range(c)], dtype=torch.int32)
+    out = run_prefill(q, kp, vp, tables, torch.tensor(short, dtype=torch.int32), cu, chunks)
+    torch.testing.assert_close(out, paged_attention_cpu(q, kp, vp, row_tables, seen), atol=atol, rtol=rtol)

@@ -26,7 +26,7 @@
 //
 // Launches with few query tiles cut the keys into segments and merge them (see
 // kSegTiles).  fp32 rows of head_dim 128 on 16 bytes, page 16, have their own
-// kernel (paged_prefill_f32.hip).
+// kernel (paged_prefill_f32.hip) where it pays (f32_kernel_pays).
 //
 // Other shapes expand each query row into a decode row (its own key length and
 // a copy of its sequence's table row) in the workspace and run the split-K
@@ -1087,6 +1087,27 @@ int max_segments(int64_t total_q, int64_t num_seqs, int64_t width, int64_t hq) {
   const int64_t by_keys = width * kPage / kBN / kSegTiles;
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({kCus / items, by_keys, kMaxSeg})));
 }
+// Whether the fp32 matrix-core kernel is taken rather than the per-token path.
+// It walks a row tile's keys in one workgroup, at the same cost for 1 row as for
+// 32, and needs 256 (row tile, head) items to fill the chip; the per-token path
+// spreads a row's keys over the chip and pays for every row.  Both costs in
+// units of 10 us, fitted to 1769 launches of 8 to 256 rows over 64 to 32768
+// keys and 4 to 64 heads: the choice is within 2% of the faster one on average
+// and at most 10% slower.  Measured (16 heads, one sequence, us, per-token
+// against kernel): 1 row over 700 keys 27.8 / 37.3, over 32768 92.7 / 1270; 16
+// over 4096 72.5 / 165; 32 over 4096 126.8 / 165; 64 over 4096 236 / 172.  32 q
+// and 8 kv heads: 8 rows over 200 keys 31 / 13, over 4096 55 / 165.
+bool f32_kernel_pays(int64_t total_q, int64_t num_seqs, int64_t max_seqlen_q, int64_t width, int64_t hq, int64_t hkv) {
+  int64_t tiles = (total_q + 31 * num_seqs) / 32;
+  if (max_seqlen_q > 0) tiles = std::min(tiles, num_seqs * ((max_seqlen_q + 31) / 32));
+  const double splits = static_cast<double>(width) * kPage / 256;  // of the widest row
+  const double rounds = std::max(1.0, static_cast<double>(tiles) * hq / kCus);
+  const int64_t group = hq / hkv;
+  const double kernel = rounds * (0.85 + std::max(0.4, splits));
+  const double tokens = 0.4 + (0.9 + 0.8 * group) * std::min(1.0, splits) +
+                        (group == 1 ? 1.36e-3 : 0.95e-3) * static_cast<double>(total_q) * hq * splits;
+  return kernel < tokens;
+}
 struct SplitLayout {
   int64_t ml, total;  // the accumulators come first
 };
@@ -1231,9 +1252,10 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
                 "requires 16-byte aligned q/out/cache rows and head_dim 64/128, page 16, bf16/fp16)",
                 (long long)workspace_bytes, (long long)need);
   if (!aligned16(workspace)) return fail(RLT_EINVAL, "rlt_paged_prefill: workspace must be 16-byte aligned");
-  if (rows_ok && dtype == RLT_FLOAT32 && head_dim == 128 && page_size == kPage) {
+  if (split && rows_ok && dtype == RLT_FLOAT32 && head_dim == 128 && page_size == kPage &&
+      f32_kernel_pays(total_q, num_seqs, max_seqlen_q, max_table_width, num_q_heads, num_kv_heads)) {
     // The fp32 matrix-core kernel; the workspace stays unused (its size is
-    // the per-token path's, which rows off 16 bytes take).
+    // the per-token path's).
     PrefillF32Args p{};
     p.q = static_cast<const float*>(q);
     p.q_row = q_strides[0];

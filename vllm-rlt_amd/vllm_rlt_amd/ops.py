@@ -635,11 +635,11 @@ def paged_prefill(
 
     The 16-bit MFMA path needs no workspace.  Other shapes need
     prefill_workspace_bytes(...) bytes: unaligned rows and other head or page
-    sizes run each query row as a decode row there (aligned fp32 rows of
-    head_dim 128, page 16 leave it unused).  They are allocated here unless `workspace`
-    (a uint8 device tensor at least that large) is given.  Without a given
-    workspace, long key ranges of short chunks are cut into segments whose
-    partials are allocated here (rlt_paged_prefill_split).
+    sizes run each query row as a decode row there (launches of enough aligned
+    fp32 rows of head_dim 128, page 16 leave it unused).  They are allocated here
+    unless `workspace` (a uint8 device tensor at least that large) is given.
+    Without a given workspace, long key ranges of short chunks are cut into
+    segments whose partials are allocated here (rlt_paged_prefill_split).
     """
     if workspace is None:
         host, stream = _host_calls(q)
@@ -659,7 +659,11 @@ def paged_prefill(
 def _paged_prefill(
     q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace, split
 ):
-    """paged_prefill; split: the workspace is this call's alone, so segment partials may go there."""
+    """paged_prefill; split: the workspace is this call's alone, so segment partials may go there.
+
+    fp32 has no segment partials and may always choose its kernel by the launch.
+    """
+    split = split or q.dtype == torch.float32
     device = _require_rocm(q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q)
     if q.ndim != 3 or key_cache.ndim != 4:
         raise ValueError("q must be [tokens, heads, head_dim] and caches [blocks, page, kv_heads, head_dim]")
