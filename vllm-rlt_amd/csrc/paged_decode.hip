@@ -8,9 +8,10 @@
 // wavefront processes one (row, kv_head, split) item.  When the kv head count
 // is a multiple of the workgroup's 4 waves, a workgroup owns one (row, split,
 // block of 4 heads) and workgroups are laid out so that each XCD serves whole
-// (split, head block) groups with all rows of a group back to back: rows whose
-// tables alias the same pages (a shared prefix) read them at the same time
-// through one L2.  Otherwise the four waves of a workgroup walk the compact
+// (split, head block) groups with all rows of a group back to back, as far as
+// the groups divide among the 8 XCDs (xcd_item): rows whose tables alias the same
+// pages (a shared prefix) read them at the same time through one L2.  The groups
+// left over are dealt out over all XCDs.  Otherwise the four waves of a workgroup walk the compact
 // item list (rows x splits x kv_heads, kv_head innermost) in grid-stride order,
 // after each workgroup builds the exclusive prefix of split counts over rows
 // in LDS; neither schedule needs host-side length information.
@@ -39,6 +40,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "decode_aliased.hpp"
 #include "mfma.hpp"
 
 // Split-K partials of rlt_paged_decode_no_alloc: a fixed per-device array in
@@ -157,6 +159,7 @@ struct DecodeArgs {
   int n_rows, hkv, hq, d, page;
   int xcd_groups;  // > 0: XCD-affine schedule over this many (split, head block) groups
   uint32_t rows_inverse, rest_inverse;  // inverse() of n_rows and of xcd_groups % kXcds
+  int rows_alias;   // nonzero: rows next to each other read the same pages
   int64_t num_blocks;
   int64_t max_len;  // table width * page: lengths are clamped to what the table covers
   float qscale;     // softmax scale * log2(e)
@@ -341,7 +344,11 @@ __device__ __forceinline__ uint32_t divide(uint32_t x, uint32_t n, uint32_t inve
 // from one L2.  Every second round runs in reverse: later splits have fewer
 // rows, and so each pair of rounds gives every XCD about the same number of
 // items.  The groups left over, fewer than kXcds, are dealt out by rows as well,
-// so that no XCD is left without work.  Measured, us, graph-timed, against
+// so that no XCD is left without work, unless the launch's rows alias each
+// other's pages (rows_alias: a prefill's rows): then each XCD takes an eighth of
+// their items, group after group, and reads the pages of two groups at most (48
+// rows of 700 tokens, 8 fp32 heads: 6 groups, 35.5 us whole on an XCD each,
+// 47.4 by rows, 38.4 so).  Measured, us, graph-timed, against
 // rounds rotated by one XCD and left-over groups whole on an XCD each: 16 kv heads,
 // rows of one split (4 groups: half the XCDs) 256 rows of 128-256 tokens 93.0 /
 // 68.5, 128 of 64-128 30.0 / 21.2, 161 of 595-724 165 / 147, 40 of 1-1300 50.4 /
@@ -363,6 +370,13 @@ __device__ __forceinline__ bool xcd_item(const DecodeArgs& a, int b, int* r, int
     return true;
   }
   if (rest == 0) return false;
+  if (a.rows_alias) {
+    const uint32_t left = rest * a.n_rows, item = x * left / kXcds + i;
+    const uint32_t group = divide(item, a.n_rows, a.rows_inverse);
+    *r = uniform(static_cast<int>(item - group * a.n_rows));
+    *gi = uniform(static_cast<int>(kXcds * rounds + group));
+    return item < (x + 1) * left / kXcds;
+  }
   const uint32_t left = i * kXcds + x;
   const uint32_t row = divide(left, rest, a.rest_inverse);
   *r = uniform(static_cast<int>(row));
@@ -2000,7 +2014,7 @@ int paged_decode(const void* q, const int64_t* q_strides, const void* key_cache,
                  const int32_t* context_lengths, void* out, const int64_t* out_strides, int64_t n_rows,
                  int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_blocks,
                  float scale, int dtype, void* workspace, int64_t workspace_bytes, void* stream,
-                 const PrefixHint* hint, const AppendSource* append = nullptr) {
+                 const PrefixHint* hint, const AppendSource* append = nullptr, bool rows_alias = false) {
   const int esize = dtype_size(dtype);
   if (!esize) return fail(RLT_EINVAL, "rlt_paged_decode: unknown dtype %d", dtype);
   if (n_rows < 0) return fail(RLT_EINVAL, "rlt_paged_decode: n_rows is negative");
@@ -2046,6 +2060,7 @@ int paged_decode(const void* q, const int64_t* q_strides, const void* key_cache,
   a.num_blocks = num_blocks;
   a.max_len = max_table_width * page_size;
   a.qscale = scale * kLog2e;
+  a.rows_alias = rows_alias;
   if (hint) {
     a.pg_row_group = hint->buffer;
     a.pg_groups = a.pg_row_group + n_rows;
@@ -2100,6 +2115,17 @@ int paged_decode(const void* q, const int64_t* q_strides, const void* key_cache,
 }
 
 }  // namespace
+
+int rlt::paged_decode_aliased(const void* q, const int64_t* q_strides, const void* key_cache, const void* value_cache,
+                              const int64_t* kv_strides, const int32_t* block_tables, int64_t table_stride,
+                              int64_t max_table_width, const int32_t* context_lengths, void* out,
+                              const int64_t* out_strides, int64_t n_rows, int64_t num_q_heads, int64_t num_kv_heads,
+                              int64_t head_dim, int64_t page_size, int64_t num_blocks, float scale, int dtype,
+                              void* workspace, int64_t workspace_bytes, void* stream) {
+  return paged_decode(q, q_strides, key_cache, value_cache, kv_strides, block_tables, table_stride, max_table_width,
+                      context_lengths, out, out_strides, n_rows, num_q_heads, num_kv_heads, head_dim, page_size,
+                      num_blocks, scale, dtype, workspace, workspace_bytes, stream, nullptr, nullptr, true);
+}
 
 extern "C" int rlt_paged_decode(const void* q, const int64_t* q_strides, const void* key_cache,
                                 const void* value_cache, const int64_t* kv_strides, const int32_t* block_tables,

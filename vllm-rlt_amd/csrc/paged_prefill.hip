@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "decode_aliased.hpp"
 #include "mfma.hpp"
 #include "prefill_f32.hpp"
 
@@ -1296,10 +1297,10 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
   hipLaunchKernelGGL(expand_rows_kernel, dim3(static_cast<unsigned>(total_q)), dim3(kThreads), 0, as_stream(stream), e);
   if (int rc = check_launch("rlt_paged_prefill(expand)")) return rc;
   char* decode_ws = ws + expand_bytes(total_q, max_table_width);
-  return rlt_paged_decode(q, q_strides, key_cache, value_cache, kv_strides, e.row_tables, width, max_table_width,
-                          e.row_lens, out, out_strides, total_q, num_q_heads, num_kv_heads, head_dim, page_size,
-                          num_blocks, scale, dtype, decode_ws, workspace_bytes - expand_bytes(total_q, max_table_width),
-                          stream);
+  return paged_decode_aliased(q, q_strides, key_cache, value_cache, kv_strides, e.row_tables, width, max_table_width,
+                              e.row_lens, out, out_strides, total_q, num_q_heads, num_kv_heads, head_dim, page_size,
+                              num_blocks, scale, dtype, decode_ws,
+                              workspace_bytes - expand_bytes(total_q, max_table_width), stream);
 }
 
 }  // namespace
