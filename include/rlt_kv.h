@@ -391,7 +391,7 @@ int rlt_paged_prefill_split(const void* q, const int64_t* q_strides, const void*
 
 /*
  * Workspace bytes rlt_paged_prefill_split needs to cut key ranges (shape-only;
- * 0 when no sequence of these shapes is cut, at most 17 MB otherwise).
+ * 0 when no sequence of these shapes can be cut, at most 17 MB otherwise).
  */
 int64_t rlt_paged_prefill_split_workspace_bytes(int64_t total_q, int64_t num_seqs,
                                                 int64_t max_table_width, int64_t num_q_heads,

@@ -236,3 +236,33 @@ def test_fp32_matrix_kernel_where_it_is_taken(hq, hkv, prefixes, chunks):
     seen = torch.tensor([max(0, n - (c - 1 - i)) for n, c in zip(short, chunks) for i in range(c)], dtype=torch.int32)
     out = run_prefill(q, kp, vp, tables, torch.tensor(short, dtype=torch.int32), cu, chunks)
     torch.testing.assert_close(out, paged_attention_cpu(q, kp, vp, row_tables, seen), atol=atol, rtol=rtol)
+
+
+@pytest.mark.parametrize(
+    "hq,prefixes,chunks,cut",
+    [
+        (8, [1217], [16], True),  # 20 key tiles, room for 3 segments and more
+        (8, [1200], [16], False),  # 19
+        (8, [1217, 1000], [16, 40], True),  # the longest sequence decides for the others
+        (16, [1700, 10], [129, 300], True),  # 29 tiles; five query tiles, room for 3
+        (16, [1292], [700], True),  # 32 tiles, halves: six query tiles of 16 heads
+        (16, [1284], [700], False),  # 31
+        (32, [0, 700, 1300], [300, 300, 300], False),  # nine query tiles of 32 heads: 256 items without a cut
+    ],
+)
+def test_keys_are_cut_where_the_merge_pays(hq, prefixes, chunks, cut):
+    from vllm_rlt_amd import ops
+
+    q, kp, vp, tables, lens, cu, row_tables, row_lengths = ragged_prefill_case(
+        torch.bfloat16, hq, 8, 128, prefixes, chunks, 41
+    )
+    args = [t.cuda() for t in (q, kp, vp, tables, lens, cu)]
+    out = ops.paged_prefill(*args, max(chunks))
+    spare = torch.empty(1, dtype=torch.uint8, device="cuda")
+    plain = ops.paged_prefill(*args, max(chunks), workspace=spare)  # a given workspace: never cut
+    # A cut rounds P against a segment's own maximum, so the two differ in last bits.
+    assert torch.equal(out, plain) != cut
+    some = torch.randperm(len(q), generator=torch.Generator().manual_seed(1))[:60]
+    atol, rtol = TOL[torch.bfloat16]
+    expect = paged_attention_cpu(q[some], kp, vp, row_tables[some], row_lengths[some])
+    torch.testing.assert_close(out.cpu()[some], expect, atol=atol, rtol=rtol)

@@ -150,7 +150,8 @@ struct PrefillArgs {
   // (max in log2 units, sum) part_ml[P * total_q + i].
   f32x4* part_acc;
   float2* part_ml;
-  int max_seg;  // segments of a sequence long enough for them
+  int max_seg;    // segments of a sequence long enough for them
+  int cut_tiles;  // key tiles of the longest sequence from which the launch is cut
 };
 
 // Rows [row0, row0 + nq) of sequence s, clamped to [0, total_q] so that an
@@ -166,11 +167,11 @@ __device__ __forceinline__ void seq_rows(const PrefillArgs& a, int s, int& row0,
 // combines the partials.  The host allows max_seg segments, as many as bring
 // the launch to one item per CU; a sequence takes them as long as a segment
 // keeps kSegTiles key tiles (4 iterations of two, ~6 us, against the ~10 us
-// that an item spends outside its loop).  One 512-token chunk over 16000 keys:
-// 194 -> 94 us in 4 segments; 100 tokens over 8192 keys 123 -> 31 us
-// in 16.  With 256 items already there nothing is cut: four 512-token
-// chunks over 8192 keys took 158 us uncut and 180 us in halves, the chip being
-// at its power limit either way.
+// that an item spends outside its loop) and its keys are worth a merge
+// (cut_tiles).  One 512-token chunk over 16000 keys: 194 -> 82 us in 4
+// segments; 100 tokens over 8192 keys 123 -> 31 us in 16.  With 256 items
+// already there nothing is cut: four 512-token chunks over 8192 keys took 158 us
+// uncut and 180 us in halves, the chip being at its power limit either way.
 constexpr int kCus = 256;
 constexpr int kSegTiles = 8;
 constexpr int kMaxSeg = 16;
@@ -178,7 +179,17 @@ constexpr int kMaxSeg = 16;
 // Key tiles of len keys.
 __device__ __forceinline__ int key_tiles(int len) { return len > 0 ? (len - 1) / kBN + 1 : 0; }
 
-// Segments of a sequence of len keys, 1 <= n <= max_seg.
+// Key tiles of the longest sequence from which a launch is cut, by the segments
+// that bring it to one item per CU.  The merge costs 4-5 us, and halves of
+// launches that nearly fill the chip gain little.  Measured, cut against uncut,
+// over 1390 launches from 1 to 1024 rows of 1 to 8 sequences, 8 to 32 heads:
+// room for 3 segments or more 0.93-1.20 at 17 tiles, 0.84-1.02 at 20, 0.59-0.86
+// at 33; room for 2 0.86-1.21 at 24, 0.82-1.14 at 33 (two of 51 above 1.07).  A
+// launch whose table is wide enough but whose sequences are not pays 1.6-2 us,
+// the merge kernel's bare launch: the host does not know the lengths.
+int cut_tiles(int room) { return room >= 3 ? 20 : 32; }
+
+// Segments of a sequence of len keys, 1 <= n <= max_seg, in a launch that is cut.
 __device__ __forceinline__ int seq_segments(int len, int max_seg) {
   return max(1, min(key_tiles(len) / kSegTiles, max_seg));
 }
@@ -248,7 +259,10 @@ __device__ __forceinline__ bool find_work(const PrefillArgs& a, void* lds, Work&
     int r0, nq;
     seq_rows(a, s, r0, nq);
     const int len = static_cast<int>(min<int64_t>(a.lens[s], max_len));
-    const int n = seq_segments(len, a.max_seg);
+    // A launch is cut when its longest sequence is worth it, since it waits for
+    // the merge of any of them.
+    const bool cut = a.max_seg > 1 && __builtin_amdgcn_ballot_w64(key_tiles(len) >= a.cut_tiles) != 0;
+    const int n = seq_segments(len, cut ? a.max_seg : 1);
     const int units = seq_units<MERGE>(nq, n);
     const uint32_t key = static_cast<uint32_t>(segment_tiles(len, n)) * kWaveSeqs + (kWaveSeqs - 1 - s);
     // Lanes past ns hold copies of the last sequence: q >= ns counts nothing.
@@ -1079,15 +1093,25 @@ namespace {
 bool mfma_shape(int64_t head_dim, int64_t page_size, int dtype) {
   return (dtype == RLT_BFLOAT16 || dtype == RLT_FLOAT16) && (head_dim == 64 || head_dim == 128) && page_size == kPage;
 }
-// Segments a launch of these shapes allows its sequences (see kSegTiles): as
-// many as bring its query tiles, at least one per sequence, to one item per
-// CU.  1 when the direct-to-LDS kernel's work list is not the ranked one.
-int max_segments(int64_t total_q, int64_t num_seqs, int64_t width, int64_t hq) {
+// Query tiles of total_q rows in num_seqs sequences, at most.
+int64_t query_tiles(int64_t total_q, int64_t num_seqs) { return (total_q + num_seqs * (kBM - 1)) / kBM; }
+
+// Segments there can be in a launch of `pairs` (sequence, query tile) pairs (see
+// kSegTiles): as many as bring it to one item per CU.  1 when the direct-to-LDS
+// kernel's work list is not the ranked one.
+int segments_room(int64_t pairs, int64_t num_seqs, int64_t width, int64_t hq) {
   if (num_seqs > kRankSeqs || hq % kXcds || width > kTablePages) return 1;
-  const int64_t items = std::max<int64_t>((total_q + kBM - 1) / kBM, num_seqs) * hq;
-  const int64_t by_keys = width * kPage / kBN / kSegTiles;
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({kCus / items, by_keys, kMaxSeg})));
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kCus / (pairs * hq), kMaxSeg)));
 }
+// Segments the keys of a row of `width` pages are enough for.
+int segments_of(int64_t width) {
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(width * kPage / kBN / kSegTiles, kMaxSeg)));
+}
+// The fewest query tiles such rows can have: the most segments.
+int64_t fewest_tiles(int64_t total_q, int64_t num_seqs) {
+  return std::max<int64_t>((total_q + kBM - 1) / kBM, num_seqs);
+}
+
 // Whether the fp32 matrix-core kernel is taken rather than the per-token path.
 // It walks a row tile's keys in one workgroup, at the same cost for 1 row as for
 // 32, and needs 256 (row tile, head) items to fill the chip; the per-token path
@@ -1139,7 +1163,8 @@ extern "C" int64_t rlt_paged_prefill_split_workspace_bytes(int64_t total_q, int6
   if (!mfma_shape(head_dim, page_size, dtype))
     return fallback_workspace(total_q, max_table_width, num_q_heads, num_kv_heads, head_dim);
   if (num_q_heads <= 0 || max_table_width <= 0 || head_dim != 128) return 0;
-  return split_layout(total_q, num_q_heads, head_dim, max_segments(total_q, num_seqs, max_table_width, num_q_heads)).total;
+  const int room = segments_room(fewest_tiles(total_q, num_seqs), num_seqs, max_table_width, num_q_heads);
+  return split_layout(total_q, num_q_heads, head_dim, std::min(room, segments_of(max_table_width))).total;
 }
 
 namespace {
@@ -1203,8 +1228,8 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
     p.qscale = std::fabs(scale) * kLog2eP;
     p.q_sign = scale < 0.f ? 0x80008000u : 0u;
     // Ranked mode: each XCD's queue holds hq/8 heads of every (sequence,
-    // query tile) pair, at most ceil(total_q / kBM) + num_seqs of them.
-    const int64_t pairs_bound = (total_q + kBM - 1) / kBM + num_seqs;
+    // query tile) pair.
+    const int64_t pairs_bound = query_tiles(total_q, num_seqs);
     const int64_t max_qt = (max_seqlen_q + kBM - 1) / kBM;
     p.total_q = static_cast<int>(total_q);
     p.ranked = num_seqs <= kRankSeqs && num_q_heads % kXcds == 0;
@@ -1215,8 +1240,16 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
     // a workgroup's query rows within 32-bit offsets).
     const bool dma = head_dim == 128 && max_table_width <= kTablePages && q_strides[0] >= 0 &&
                      q_strides[0] * esize * kBM < (int64_t(1) << 31);
-    // Key segments, when the caller gave room for their partials.
-    p.max_seg = split && dma && p.ranked ? max_segments(total_q, num_seqs, max_table_width, num_q_heads) : 1;
+    // Key segments, when the caller gave room for their partials.  Sequences
+    // are expected to be no longer than max_seqlen_q says.
+    const int64_t pairs = std::max(fewest_tiles(total_q, num_seqs),
+                                   max_qt > 0 ? std::min(pairs_bound, num_seqs * max_qt) : pairs_bound);
+    const int room = split && dma && p.ranked ? segments_room(pairs, num_seqs, max_table_width, num_q_heads) : 1;
+    const bool may_cut = (max_table_width * kPage + kBN - 1) / kBN >= cut_tiles(room);
+    p.max_seg = may_cut ? std::min(room, segments_of(max_table_width)) : 1;
+    // The table does not say how long the sequences are: once the merge has to
+    // be launched, less keys are worth a cut (100 rows over 1000 keys 25.1 / 21.5 us).
+    p.cut_tiles = cut_tiles(room) - 4;
     const SplitLayout layout = split_layout(total_q, num_q_heads, head_dim, p.max_seg);
     if (p.max_seg > 1 && workspace && aligned16(workspace) && workspace_bytes >= layout.total) {
       p.part_acc = static_cast<f32x4*>(workspace);
