@@ -159,6 +159,35 @@ def test_calls_left_to_python():
         )
 
 
+@pytest.mark.parametrize("n_write", [3, 1 << 40, 1 << 63, 1 << 70])
+def test_an_append_of_more_rows_than_there_are_is_refused(n_write):
+    from vllm_rlt_amd import ops
+    from vllm_rlt_amd.paged_attention import HipPagedAttention
+
+    case = random_decode_case([20, 40], hq=4, hkv=4, d=128, dtype=torch.bfloat16, seed=1).to("cuda")
+    args = (case.q, case.key_slice, case.value_slice, case.tables, case.lengths, *decode_args(case))
+    with pytest.raises(ValueError, match="n_write"):
+        ops.paged_decode_append(*args, n_write=n_write)
+    attention = HipPagedAttention("cuda", torch.bfloat16, 128, 16)
+    attention.reserve_decode(2, 4, 4)
+    with pytest.raises(ValueError, match="n_write"):
+        attention.decode_append(*args, n_write=n_write)
+
+
+def test_prefill_on_the_attention_objects_workspace():
+    from vllm_rlt_amd.paged_attention import HipPagedAttention
+
+    for dtype, d in ((torch.bfloat16, 128), (torch.float32, 128), (torch.bfloat16, 256)):
+        chunks = [40, 3]
+        q, kp, vp, tables, lens, cu, _, _ = ragged_prefill_case(dtype, 8, 8, d, [100, 0], chunks, 5)
+        args = [t.cuda() for t in (q, kp, vp, tables, lens, cu)]
+        attention = HipPagedAttention("cuda", dtype, d, 16)
+        first = attention.prefill(*args, max(chunks))  # reserves the workspace, if the path needs one
+        if attention.workspace_bytes == 0:
+            attention.reserve(1)
+        assert torch.equal(direct(lambda: attention.prefill(*args, max(chunks)), "prefill"), first)
+
+
 def test_side_stream_and_capture():
     from vllm_rlt_amd.paged_attention import HipPagedAttention
 

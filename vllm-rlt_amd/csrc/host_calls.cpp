@@ -124,6 +124,10 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (args[13] == Py_None) n = app[2]->size(0);
     else if (PyLong_CheckExact(args[13])) n = PyLong_AsLongLong(args[13]);
     else Py_RETURN_NONE;
+    if (PyErr_Occurred()) {  // n_write past 64 bits
+      PyErr_Clear();
+      Py_RETURN_NONE;
+    }
     if (n < 0 || n > rows || n > app[2]->size(0) || n > app[3]->size(0)) Py_RETURN_NONE;
     for (int i = 0; i < 2; ++i)
       if (app[i]->dim() != 3 || app[i]->size(1) != hkv || app[i]->size(2) != d || app[i]->size(0) < n ||
