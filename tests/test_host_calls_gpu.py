@@ -188,6 +188,21 @@ def test_prefill_on_the_attention_objects_workspace():
         assert torch.equal(direct(lambda: attention.prefill(*args, max(chunks)), "prefill"), first)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_attention_object_without_host_calls(python_path, dtype):
+    from vllm_rlt_amd.paged_attention import HipPagedAttention
+
+    case = random_decode_case([1, 33, 300, 700], hq=8, hkv=8, d=128, dtype=dtype, seed=3).to("cuda")
+    decode = (case.q, case.key_slice, case.value_slice, case.tables, case.lengths)
+    append = (*decode, *decode_args(case))
+    q, kp, vp, tables, lens, cu, _, _ = ragged_prefill_case(dtype, 8, 8, 128, [100, 0], [40, 3], 5)
+    prefill = [t.cuda() for t in (q, kp, vp, tables, lens, cu)]
+    attention = HipPagedAttention("cuda", dtype, 128, 16)
+    attention.reserve_decode(4, 8, 8)
+    for run in (lambda: attention(*decode), lambda: attention.decode_append(*append), lambda: attention.prefill(*prefill, 40)):
+        assert torch.equal(python_path(run), run())
+
+
 def test_side_stream_and_capture():
     from vllm_rlt_amd.paged_attention import HipPagedAttention
 

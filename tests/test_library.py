@@ -2,9 +2,13 @@
 
 import ctypes
 import re
+import subprocess
+import sys
+from pathlib import Path
 
 import pytest
 
+import vllm_rlt_amd
 from conftest import REPO
 
 
@@ -134,3 +138,36 @@ def test_int64_arrays_are_shared_by_value():
     assert list(strides) == [2048, 128, 1]
     assert list(_native.int64_array(list(range(20)))) == list(range(20))
     assert list(_native.int64_array([])) == []
+
+
+def test_library_loads_without_the_host_calls(monkeypatch):
+    _, native = _library()
+    monkeypatch.setattr(native, "_lib", None)
+    monkeypatch.setattr(native, "host", None)
+    monkeypatch.setitem(sys.modules, "vllm_rlt_amd._host_calls", None)  # an import of it fails
+    monkeypatch.delattr(vllm_rlt_amd, "_host_calls", raising=False)
+    with pytest.warns(UserWarning, match="host calls cannot be used"):
+        lib = native.load()
+    assert lib.rlt_version() and native.host is None
+
+
+def test_library_builds_without_the_host_calls(monkeypatch, tmp_path):
+    from vllm_rlt_amd import _build
+
+    def no_compiler():
+        raise FileNotFoundError("g++")
+
+    def run(cmd, **kw):
+        Path(cmd[cmd.index("-o") + 1]).touch()
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(_build, "build_host_calls", no_compiler)
+    monkeypatch.setattr(_build, "_compile", lambda source: tmp_path / source.stem)
+    monkeypatch.setattr(_build, "hipcc", lambda: "hipcc")
+    monkeypatch.setattr(_build.subprocess, "run", run)
+    monkeypatch.setattr(_build, "LIBRARY", tmp_path / "librlt_kv.so")
+    monkeypatch.setattr(_build, "HOST_CALLS", tmp_path / "_host_calls.so")
+    (tmp_path / "_host_calls.so").touch()  # one of an earlier build
+    with pytest.warns(UserWarning, match="not built"):
+        assert _build.build() == tmp_path / "librlt_kv.so"
+    assert not (tmp_path / "_host_calls.so").exists()

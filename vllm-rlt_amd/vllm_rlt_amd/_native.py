@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import warnings
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
@@ -142,8 +143,9 @@ SIGNATURES = {
 }
 
 _lib = None
-# The extension module of csrc/host_calls.cpp, bound to the loaded library:
-# the hot calls from tensors to the C ABI without ctypes (None before load()).
+# The extension module of csrc/host_calls.cpp, bound to the loaded library: the
+# hot calls from tensors to the C ABI without ctypes (None before load(), and
+# where the module cannot be used).
 host = None
 
 
@@ -157,6 +159,18 @@ HOST_CALLED = (
     "rlt_paged_prefill_workspace_bytes",
     "rlt_rope_kv_append",
 )
+
+
+def _bind_host_calls(lib):
+    """The host calls bound to lib; None, with a warning, where they cannot be used (not built, another torch)."""
+    try:
+        from . import _host_calls
+
+        _host_calls.bind(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in HOST_CALLED))
+    except (ImportError, TypeError) as error:
+        warnings.warn(f"the C++ host calls cannot be used, every call goes through Python (slower): {error}", stacklevel=3)
+        return None
+    return _host_calls
 
 
 def load(path: Path | str = LIBRARY_PATH) -> ctypes.CDLL:
@@ -175,15 +189,7 @@ def load(path: Path | str = LIBRARY_PATH) -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = restype
         fn.argtypes = argtypes
-    try:
-        from . import _host_calls
-    except ImportError as error:
-        raise RuntimeError(
-            f"the host calls beside {path.name} are missing: build the package first (python __graft_entry__.py build "
-            "or python -m vllm_rlt_amd._build)"
-        ) from error
-    _host_calls.bind(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in HOST_CALLED))
-    host = _host_calls
+    host = _bind_host_calls(lib)
     _lib = lib
     return lib
 

@@ -112,6 +112,8 @@ class HipPagedAttention:
         if workspace is None or not q.is_cuda:
             return None
         host, stream = ops._host_calls(q)
+        if host is None:
+            return None
         out = host.decode(
             q, key_cache, value_cache, block_tables, context_lengths, None, workspace, None, stream, *append
         )
@@ -162,12 +164,13 @@ class HipPagedAttention:
         # Under capture the steps below note that a graph reads the workspace.
         if self._workspace is not None and q.is_cuda and not torch._C._cuda_isCurrentStreamCapturing():
             host, stream = ops._host_calls(q)
-            out = host.prefill(
-                q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None, stream,
-                self._workspace,
-            )
-            if out is not None:
-                return ops._finish(out, "rlt_paged_prefill")
+            if host is not None:
+                out = host.prefill(
+                    q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None,
+                    stream, self._workspace,
+                )
+                if out is not None:
+                    return ops._finish(out, "rlt_paged_prefill")
         need = ops.prefill_workspace_bytes(
             q.shape[0], block_tables.shape[0], block_tables.shape[1], q.shape[1], key_cache.shape[2], self.head_dim,
             self.block_size, q.dtype if ops.rows_aligned16(q, key_cache, value_cache) else torch.float32,
