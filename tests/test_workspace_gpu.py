@@ -151,3 +151,42 @@ def test_workspace_batch_writes_and_attends_like_the_manager(layout):
     ws.release()
     ws.acquire()
     assert ws.event is not None and ws.event.query()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_steady_state_prefill_allocates_its_result_only(dtype):
+    # One chunk over a long prefix: its key segments live in the object's workspace,
+    # which the plan for as many rows covers.
+    from vllm_rlt_amd import ops
+    from vllm_rlt_amd.paged_attention import HipPagedAttention
+
+    rows, heads, pages = 300, 8, 400
+    kv = [torch.randn(pages, 16, heads, 128, device="cuda", dtype=dtype) for _ in range(2)]
+    q = torch.randn(rows, heads, 128, device="cuda", dtype=dtype)
+    tables = torch.randperm(pages, device="cuda").int()[None]
+    lens = torch.tensor([16 * pages - 5], dtype=torch.int32, device="cuda")
+    cu = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    need = ops.prefill_split_workspace_bytes(rows, 1, pages, heads, heads, 128, 16, dtype)
+    assert need > 0
+    attention = HipPagedAttention("cuda", dtype, 128, 16)
+    first = attention.prefill(q, *kv, tables, lens, cu, rows)
+    assert attention.workspace_bytes >= need
+    plan = max(ops.decode_workspace_bytes(rows, heads, heads, 128),
+               ops.prefill_workspace_bytes(rows, 1, pages, heads, heads, 128, 16, dtype))
+    assert attention.workspace_bytes <= HipPagedAttention.workspace_size_for(plan)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = attention.prefill(q, *kv, tables, lens, cu, rows)
+    assert torch.cuda.max_memory_allocated() - before == out.numel() * out.element_size()
+    assert torch.equal(out, first)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = attention.prefill(q, *kv, tables, lens, cu, rows)
+    for _ in range(3):
+        q.normal_()
+        graph.replay()
+        assert torch.equal(captured, attention.prefill(q, *kv, tables, lens, cu, rows))
+    held = attention.workspace_bytes
+    attention.reserve(held + 1)
+    assert attention.held_bytes == held  # the graph keeps the workspace it reads

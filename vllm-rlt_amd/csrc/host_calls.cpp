@@ -32,7 +32,6 @@ decltype(&rlt_paged_decode_append) g_decode_append = nullptr;
 decltype(&rlt_paged_decode_workspace_bytes) g_decode_bytes = nullptr;
 decltype(&rlt_paged_prefill_split) g_prefill = nullptr;
 decltype(&rlt_paged_prefill_split_workspace_bytes) g_prefill_bytes = nullptr;
-decltype(&rlt_paged_prefill_workspace_bytes) g_prefill_required = nullptr;
 decltype(&rlt_rope_kv_append) g_rope = nullptr;
 
 // A plain device tensor of torch.Tensor itself, or null.  (Parameters and other
@@ -168,9 +167,8 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // prefill(q, key, value, tables, lengths, cu, max_seqlen_q, out, scale, stream,
-//         workspace): the workspace the shapes need (fp32, rows off 16 bytes and
-// other per-token shapes) is the given one when it is large enough and
-// allocated here for None; room for key segments is always allocated here.
+//         workspace): the workspace for key segments or the per-token path is the
+// given one when it is large enough, allocated here for None.
 PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs != 11 || modes_active()) Py_RETURN_NONE;
@@ -194,17 +192,13 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // Rows off 16 bytes take the per-token path, whose workspace is the fp32 one's.
   const bool rows16 = aligned_rows(q) && aligned_rows(out) && aligned_rows(k) && aligned_rows(v);
   const int sized = rows16 ? code : int{RLT_FLOAT32};
+  const int64_t need = g_prefill_bytes(total, nseq, tables.size(1), hq, hkv, d, k.size(1), sized);
   at::Tensor workspace;
   if (args[10] != Py_None) {
-    const int64_t required = g_prefill_required(total, nseq, tables.size(1), hq, hkv, d, k.size(1), sized);
-    if (required > 0) {
-      const at::Tensor* w = plain(args[10]);
-      if (!w || w->scalar_type() != at::kByte || w->device() != q.device() || w->numel() < required) Py_RETURN_NONE;
-      workspace = *w;
-    }
-  }
-  if (!workspace.defined()) {
-    const int64_t need = g_prefill_bytes(total, nseq, tables.size(1), hq, hkv, d, k.size(1), sized);
+    const at::Tensor* w = plain(args[10]);
+    if (!w || w->scalar_type() != at::kByte || w->device() != q.device() || w->numel() < need) Py_RETURN_NONE;
+    workspace = *w;
+  } else {
     workspace = at::empty({need > 0 ? need : 1}, q.options().dtype(at::kByte));
   }
   void* const stream = PyLong_AsVoidPtr(args[9]);
@@ -268,13 +262,13 @@ PyObject* rope(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(decode, decode_append, decode_bytes, prefill, prefill_bytes, prefill_required, rope):
+// bind(decode, decode_append, decode_bytes, prefill, prefill_bytes, rope):
 // addresses of the loaded library's entry points.
 PyObject* bind(PyObject*, PyObject* args) {
-  PyObject* a[7];
-  if (!PyArg_ParseTuple(args, "OOOOOOO", &a[0], &a[1], &a[2], &a[3], &a[4], &a[5], &a[6])) return nullptr;
-  void* p[7];
-  for (int i = 0; i < 7; ++i) {
+  PyObject* a[6];
+  if (!PyArg_ParseTuple(args, "OOOOOO", &a[0], &a[1], &a[2], &a[3], &a[4], &a[5])) return nullptr;
+  void* p[6];
+  for (int i = 0; i < 6; ++i) {
     p[i] = PyLong_AsVoidPtr(a[i]);
     if (!p[i] && PyErr_Occurred()) return nullptr;
   }
@@ -283,8 +277,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   g_decode_bytes = reinterpret_cast<decltype(g_decode_bytes)>(p[2]);
   g_prefill = reinterpret_cast<decltype(g_prefill)>(p[3]);
   g_prefill_bytes = reinterpret_cast<decltype(g_prefill_bytes)>(p[4]);
-  g_prefill_required = reinterpret_cast<decltype(g_prefill_required)>(p[5]);
-  g_rope = reinterpret_cast<decltype(g_rope)>(p[6]);
+  g_rope = reinterpret_cast<decltype(g_rope)>(p[5]);
   Py_RETURN_NONE;
 }
 

@@ -156,7 +156,6 @@ HOST_CALLED = (
     "rlt_paged_decode_workspace_bytes",
     "rlt_paged_prefill_split",
     "rlt_paged_prefill_split_workspace_bytes",
-    "rlt_paged_prefill_workspace_bytes",
     "rlt_rope_kv_append",
 )
 

@@ -10,8 +10,9 @@ allocated next to the pool, asking each allocating object for its size:
 
 * the attention backend's grow-only workspace at its final size
   (HipPagedAttention.workspace_size_for over rlt_paged_decode_workspace_bytes
-  for the largest decode batch and rlt_paged_prefill_workspace_bytes for the
-  per-token prefill path, which the pool's dtype and shape decide), and with
+  for the largest decode batch, rlt_paged_prefill_workspace_bytes for the
+  per-token prefill path, which the pool's dtype and shape decide; a prefill's
+  key segments need less than the decode batch), and with
   graphs the outgrown workspaces captured graphs keep alive (less than the
   largest graph's workspace: powers of two below it);
 * the library's static device array (rlt_static_device_bytes);
@@ -94,7 +95,8 @@ def execution_bytes(config, scheduler, cache, execution, element_size: int, num_
     planes = config.total_ut_steps if cache.layout == "last_exited" else 1
     heads = num_q_heads or config.num_attention_heads
     costs = {}
-    # One backend workspace serves decode partials and the per-token prefill path.
+    # One backend workspace serves decode partials (64 splits a row), a prefill's key
+    # segments (at most 16 a row: never more) and the per-token prefill path.
     decode = ops.decode_workspace_bytes(rows, heads, config.num_key_value_heads, config.head_dim)
     # Zero on the MFMA prefill path; the per-token path's rows otherwise.
     prefill = ops.prefill_workspace_bytes(

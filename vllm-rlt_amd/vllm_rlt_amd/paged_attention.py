@@ -33,8 +33,8 @@ class HipPagedAttention:
     """Attention backend object for KVCacheManager(backend="hip").
 
     The object owns one grow-only device workspace for the decode split
-    partials and the per-token prefill path, so steady-state calls allocate
-    nothing.  It grows to the next power of two when a batch needs more
+    partials, a prefill's key segments and the per-token prefill path, so
+    steady-state calls allocate nothing but their result.  It grows to the next power of two when a batch needs more
     (reserve() grows it ahead of a graph capture).  A buffer it outgrows is
     released, unless a graph was captured while it was the workspace: such a
     graph keeps reading that address, so the buffer stays alive with the
@@ -171,11 +171,12 @@ class HipPagedAttention:
                 )
                 if out is not None:
                     return ops._finish(out, "rlt_paged_prefill")
-        need = ops.prefill_workspace_bytes(
+        dtype = q.dtype if ops.rows_aligned16(q, key_cache, value_cache) else torch.float32
+        need = ops.prefill_split_workspace_bytes(
             q.shape[0], block_tables.shape[0], block_tables.shape[1], q.shape[1], key_cache.shape[2], self.head_dim,
-            self.block_size, q.dtype if ops.rows_aligned16(q, key_cache, value_cache) else torch.float32,
+            self.block_size, dtype,
         )
-        workspace = self.reserve(need) if need else None
-        return ops.paged_prefill(
-            q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, workspace=workspace
+        return ops._paged_prefill(
+            q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None,
+            self.reserve(need) if need else None, True,
         )
