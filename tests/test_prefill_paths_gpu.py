@@ -266,3 +266,24 @@ def test_keys_are_cut_where_the_merge_pays(hq, prefixes, chunks, cut):
     atol, rtol = TOL[torch.bfloat16]
     expect = paged_attention_cpu(q[some], kp, vp, row_tables[some], row_lengths[some])
     torch.testing.assert_close(out.cpu()[some], expect, atol=atol, rtol=rtol)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_batch_invariant_rows_keep_their_bits_in_any_launch(dtype):
+    from vllm_rlt_amd import ops
+    from vllm_rlt_amd.paged_attention import HipPagedAttention
+
+    prefixes, chunks = [3000, 100, 900, 0], [40, 300, 200, 500]
+    q, kp, vp, tables, lens, cu, _, _ = ragged_prefill_case(dtype, 16, 16, 128, prefixes, chunks, 43)
+    q, kp, vp, tables, lens, cu = (t.cuda() for t in (q, kp, vp, tables, lens, cu))
+    one = torch.tensor([0, chunks[0]], dtype=torch.int32, device="cuda")
+    alone = (q[: chunks[0]], kp, vp, tables[:1], lens[:1], one, chunks[0])
+    together = (q, kp, vp, tables, lens, cu, max(chunks))
+    attention = HipPagedAttention("cuda", dtype, 128, 16, batch_invariant=True)
+    for call in (lambda *a: ops.paged_prefill(*a, batch_invariant=True), attention.prefill):
+        assert torch.equal(call(*alone), call(*together)[: chunks[0]])
+    attention.batch_invariant = False
+    for call in (ops.paged_prefill, attention.prefill):  # what it is an option for
+        assert not torch.equal(call(*alone), call(*together)[: chunks[0]])
+        atol, rtol = TOL[dtype]
+        torch.testing.assert_close(call(*alone), call(*together)[: chunks[0]], atol=atol, rtol=rtol)

@@ -630,6 +630,7 @@ def paged_prefill(
     out: torch.Tensor | None = None,
     scale: float | None = None,
     workspace: torch.Tensor | None = None,
+    batch_invariant: bool = False,
 ) -> torch.Tensor:
     """Packed bottom-right-causal prefill (FlashPagedAttention.prefill, flash_attention.py:66-96).
 
@@ -640,8 +641,13 @@ def paged_prefill(
     unless `workspace` (a uint8 device tensor at least that large) is given.
     Without a given workspace, long key ranges of short chunks are cut into
     segments whose partials are allocated here (rlt_paged_prefill_split).
+
+    Cut keys and the kernel of fp32 rows are chosen by the launch's shapes, so a
+    row's last bits may depend on what shares its launch.  With `batch_invariant`
+    they depend on its own sequence only (rlt_paged_prefill): no keys are cut, and
+    fp32 rows take the per-token path.
     """
-    if workspace is None:
+    if workspace is None and not batch_invariant:
         host, stream = _host_calls(q)
         if host is not None:
             result = host.prefill(
@@ -650,20 +656,17 @@ def paged_prefill(
             )
             if result is not None:
                 return _finish(result, "rlt_paged_prefill")
+    # fp32 has no segment partials: its kernel may be chosen on a given workspace too.
+    split = not batch_invariant and (workspace is None or q.dtype == torch.float32)
     return _paged_prefill(
-        q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace,
-        workspace is None,
+        q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace, split
     )
 
 
 def _paged_prefill(
     q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, out, scale, workspace, split
 ):
-    """paged_prefill; split: the workspace is this call's alone, so segment partials may go there.
-
-    fp32 has no segment partials and may always choose its kernel by the launch.
-    """
-    split = split or q.dtype == torch.float32
+    """paged_prefill; split: by rlt_paged_prefill_split, segment partials in the workspace."""
     device = _require_rocm(q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q)
     if q.ndim != 3 or key_cache.ndim != 4:
         raise ValueError("q must be [tokens, heads, head_dim] and caches [blocks, page, kv_heads, head_dim]")

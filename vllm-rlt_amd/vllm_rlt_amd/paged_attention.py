@@ -42,12 +42,16 @@ class HipPagedAttention:
     final workspace again (powers of two below it).  Calls on one object are
     meant to run on one stream, in order: two streams sharing the object at
     once would share the workspace.
+
+    A decode row's bits depend on the row only.  A prefill row's last bits may
+    depend on what shares its launch; with `batch_invariant` they depend on its
+    own sequence only, at the speed of launches that are not cut (ops.paged_prefill).
     """
 
     generation = None
     supports_packed_prefill = True
 
-    def __init__(self, device, dtype, head_dim, block_size):
+    def __init__(self, device, dtype, head_dim, block_size, batch_invariant=False):
         device = torch.device(device)
         if device.type != "cuda" or not torch.version.hip:
             raise ValueError("the hip attention backend requires a ROCm device")
@@ -61,6 +65,7 @@ class HipPagedAttention:
         self.device = device
         self.head_dim = head_dim
         self.block_size = block_size
+        self.batch_invariant = batch_invariant
         self._workspace = None
         self._captured = False  # a graph was captured reading the current workspace
         self._held = []  # outgrown workspaces a captured graph still reads
@@ -154,6 +159,13 @@ class HipPagedAttention:
             n_write=n_write, workspace=workspace, shared_prefix=shared_prefix,
         )
 
+    def _prefill_shape(self, q, key_cache, value_cache, block_tables):
+        """The workspace queries' arguments (rows off 16 bytes are sized as fp32's, for the per-token path)."""
+        return (
+            q.shape[0], block_tables.shape[0], block_tables.shape[1], q.shape[1], key_cache.shape[2], self.head_dim,
+            self.block_size, q.dtype if ops.rows_aligned16(q, key_cache, value_cache) else torch.float32,
+        )
+
     def prefill(self, q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q):
         """Packed ragged chunks over paged prefixes, bottom-right causal.
 
@@ -161,6 +173,12 @@ class HipPagedAttention:
         end at its last query, so query i of an n_q-token chunk sees
         context_lengths[s] - (n_q - 1 - i) keys (flash_attention.py:76-80).
         """
+        if self.batch_invariant:
+            need = ops.prefill_workspace_bytes(*self._prefill_shape(q, key_cache, value_cache, block_tables))
+            return ops.paged_prefill(
+                q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q,
+                workspace=self.reserve(need) if need else None, batch_invariant=True,
+            )
         # Under capture the steps below note that a graph reads the workspace.
         if self._workspace is not None and q.is_cuda and not torch._C._cuda_isCurrentStreamCapturing():
             host, stream = ops._host_calls(q)
@@ -171,11 +189,7 @@ class HipPagedAttention:
                 )
                 if out is not None:
                     return ops._finish(out, "rlt_paged_prefill")
-        dtype = q.dtype if ops.rows_aligned16(q, key_cache, value_cache) else torch.float32
-        need = ops.prefill_split_workspace_bytes(
-            q.shape[0], block_tables.shape[0], block_tables.shape[1], q.shape[1], key_cache.shape[2], self.head_dim,
-            self.block_size, dtype,
-        )
+        need = ops.prefill_split_workspace_bytes(*self._prefill_shape(q, key_cache, value_cache, block_tables))
         return ops._paged_prefill(
             q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None,
             self.reserve(need) if need else None, True,
