@@ -634,11 +634,11 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     return pre;
   };
   // One (row r, kv head h, split sp) item per wave (per workgroup: QUAD).
-  // first_entry: QUAD's and ROW's page ids of this wave's first 64 pages when
-  // early; qi: ROW's quarter of the row, whose state it leaves in LDS.
+  // first_entry: QUAD's and ROW's page ids of this wave's quarter; qi: ROW's
+  // quarter of the row, whose state it leaves in LDS.
+  constexpr bool kShared = QUAD || ROW;  // the workgroup's waves take a quarter each
   auto process = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns,
-                     const bool early = false, const int first_entry = 0, const int qi = 0,
-                     const ItemLoads& pre = {}) {
+                     const int first_entry = 0, const int qi = 0, const ItemLoads& pre = {}) {
     if (len <= 0) {
       if (QUAD && wave != 0) return;
       if (g == 0) {
@@ -650,20 +650,18 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       store_new_token(r, h);
       return;
     }
-    const bool quartered = ROW || (kQuarters && ns <= kQuarterSplits);
-    if (QUAD && !quartered && wave != 0) return;
-    const bool shared = (QUAD || ROW) && quartered;  // by the workgroup's waves
+    const bool quartered = kShared || (kQuarters && ns <= kQuarterSplits);
     const int quarter = quartered ? split_len / kWaves : split_len;
-    const int t_begin = ROW ? qi * quarter : sp * split_len + (shared ? wave * quarter : 0);
+    const int t_begin = ROW ? qi * quarter : sp * split_len + (kShared ? wave * quarter : 0);
     if (ROW && t_begin >= len) return;
-    const int t_end = min(len, t_begin + (shared ? quarter : split_len));
+    const int t_end = min(len, t_begin + (kShared ? quarter : split_len));
     const int last = t_end - 1;
     // Fused append: the row's write slot, read up front when this is its last split.
     int64_t wb = -1, wo = -1;
     if constexpr (APPEND) {
       if (t_end == len && r < a.n_write) {
-        wb = QUAD || ROW ? pre.wb : a.write_blocks[r];
-        wo = QUAD || ROW ? pre.wo : a.write_offsets[r];
+        wb = kShared ? pre.wb : a.write_blocks[r];
+        wo = kShared ? pre.wo : a.write_offsets[r];
       }
     }
 
@@ -673,7 +671,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       const T* qrow = static_cast<const T*>(a.q) + r * a.q_row + static_cast<int64_t>(h) * G * a.q_head + lane_dim;
 #pragma unroll
       for (int j = 0; j < G; ++j) {
-        const u32x4 p = QUAD || ROW ? pre.q : *reinterpret_cast<const u32x4*>(qrow + j * a.q_head);
+        const u32x4 p = kShared ? pre.q : *reinterpret_cast<const u32x4*>(qrow + j * a.q_head);
         PK::unpack(p, qv[j]);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) qv[j][e] *= a.qscale;
@@ -706,8 +704,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
     };
     // One wave walking all quarters: after the tile that ends one.
     auto end_tile = [&](int t0) {
-      if constexpr (kQuarters) {
-        if (shared) return;
+      if constexpr (kQuarters && !kShared) {
         if (((t0 + TILE - t_begin) & (quarter - 1)) == 0 || t0 + TILE >= t_end) {
           if (t0 - t_begin < quarter) {  // the first quarter: folding it into nothing is a copy
 #pragma unroll
@@ -790,7 +787,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       const int chunk_page = c0 / P;
       const int chunk_last = (c1 - 1) / P - chunk_page;  // <= 63
       int table_entry;
-      if (shared && early) table_entry = first_entry;  // a quarter is one chunk then
+      if constexpr (kShared) table_entry = first_entry;  // a quarter is one chunk
       else table_entry = lane <= chunk_last ? trow[chunk_page + lane] : 0;
       auto tile_pages = [&](int t0, int64_t (&blk)[PPT]) {
         const int rel0 = (t0 - c0) / P;
@@ -844,36 +841,35 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       }
       u32x4 kp[NI], vp[NI];
       int64_t blk[PPT];
-      if constexpr (QUAD || ROW) {
-        if (shared && quarter == 2 * TILE) {
-          // Both tiles of a 64-token quarter in flight at once.  A second tile
-          // past the end re-reads the last token, whose V need not be finite,
-          // and is not used.
-          u32x4 kp2[NI], vp2[NI];
-          int64_t blk2[PPT];
-          tile_pages(c0, blk);
-          tile_pages(c0 + TILE, blk2);
-          if (APPEND && fresh) {
-            issue_fresh(kp, kbase, kn_row, blk, c0);
-            issue_fresh(kp2, kbase, kn_row, blk2, c0 + TILE);
-            issue_fresh(vp, vbase, vn_row, blk, c0);
-            issue_fresh(vp2, vbase, vn_row, blk2, c0 + TILE);
-          } else {
-            issue(kp, kbase, blk, c0);
-            issue(kp2, kbase, blk2, c0 + TILE);
-            issue(vp, vbase, blk, c0);
-            issue(vp2, vbase, blk2, c0 + TILE);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          float sc[G][NI];
-          scores(kp, c0, sc);
-          accumulate(vp, c0, sc);
-          if (c0 + TILE < t_end) {
-            scores(kp2, c0 + TILE, sc);
-            accumulate(vp2, c0 + TILE, sc);
-          }
-          continue;
+      if constexpr (kShared) {
+        static_assert(!kShared || kSplitTokens / kWaves == 2 * TILE, "two tiles a quarter");
+        // Both tiles of a 64-token quarter in flight at once.  A second tile
+        // past the end re-reads the last token, whose V need not be finite,
+        // and is not used.
+        u32x4 kp2[NI], vp2[NI];
+        int64_t blk2[PPT];
+        tile_pages(c0, blk);
+        tile_pages(c0 + TILE, blk2);
+        if (APPEND && fresh) {
+          issue_fresh(kp, kbase, kn_row, blk, c0);
+          issue_fresh(kp2, kbase, kn_row, blk2, c0 + TILE);
+          issue_fresh(vp, vbase, vn_row, blk, c0);
+          issue_fresh(vp2, vbase, vn_row, blk2, c0 + TILE);
+        } else {
+          issue(kp, kbase, blk, c0);
+          issue(kp2, kbase, blk2, c0 + TILE);
+          issue(vp, vbase, blk, c0);
+          issue(vp2, vbase, blk2, c0 + TILE);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        float sc[G][NI];
+        scores(kp, c0, sc);
+        accumulate(vp, c0, sc);
+        if (c0 + TILE < t_end) {
+          scores(kp2, c0 + TILE, sc);
+          accumulate(vp2, c0 + TILE, sc);
+        }
+        continue;  // one quarter, one chunk
       }
       // sched_barrier keeps every K load of a tile ahead of its V loads in
       // issue order, so waiting for K never waits for V.
@@ -925,17 +921,15 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       return;
     }
     if constexpr (QUAD) {
-      if (shared) {
-        // Wave 0 folds the quarters in order; the others hand theirs over.
-        if (wave > 0) put_state(wave - 1, m, l, acc);
-        __syncthreads();  // and every read of the item's pages is done
-        if (wave > 0) return;
-        fold(m, l, acc);
+      // Wave 0 folds the quarters in order; the others hand theirs over.
+      if (wave > 0) put_state(wave - 1, m, l, acc);
+      __syncthreads();  // and every read of the item's pages is done
+      if (wave > 0) return;
+      fold(m, l, acc);
 #pragma unroll
-        for (int w = 0; w < kWaves - 1; ++w) {
-          get_state(w, m, l, acc);
-          fold(m, l, acc);
-        }
+      for (int w = 0; w < kWaves - 1; ++w) {
+        get_state(w, m, l, acc);
+        fold(m, l, acc);
       }
     }
     if constexpr (kQuarters) {
@@ -1218,7 +1212,7 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
       return;
     }
 #pragma unroll
-    for (int i = 0; i < kRounds; ++i) process(r, h, 0, len, kSplitTokens, ns, true, entry[i], wave + kRowWaves * i, pre);
+    for (int i = 0; i < kRounds; ++i) process(r, h, 0, len, kSplitTokens, ns, entry[i], wave + kRowWaves * i, pre);
     __syncthreads();  // every quarter is in LDS, every page has been read
     if (wave == kRowWaves - 1) store_new_token(r, h);
     float m[G], l[G], acc[G][EPL];
@@ -1273,22 +1267,20 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   }
   if constexpr (QUAD) {
     // One (row, split, head) per workgroup, laid out as the XCD-affine
-    // schedule below with heads in place of head blocks.  The row's length, q,
-    // the write slot and, when the split length does not depend on the row's
-    // own, its page ids go out together.
+    // schedule with heads in place of head blocks.  The table spans at most
+    // kQuarterSplits splits, so the split length is kSplitTokens and the row's
+    // length, q, the write slot and its page ids go out together.
     int r, gi;
     if (!xcd_item(a, block, &r, &gi)) return;
     const int sp = gi / a.hkv;
     const int h = gi - sp * a.hkv;
-    const bool early = a.max_len <= kMaxSplits * kSplitTokens;
     const int page0 = sp * (kSplitTokens / P) + wave * (kSplitTokens / P / kWaves);
     const int width = static_cast<int>(a.max_len / P);
-    const int entry = early && width > 0 ? a.tables[r * a.table_stride + min(page0 + (lane & 3), width - 1)] : 0;
+    const int entry = a.tables[r * a.table_stride + min(page0 + (lane & 3), width - 1)];
     const ItemLoads pre = load_item(r, h);
     const int len = uniform(row_length(a, r));
-    int split_len, ns;
-    split_plan(len, &split_len, &ns);
-    if (sp < ns) process(r, h, sp, len, split_len, ns, early, entry, 0, pre);
+    const int ns = len > 0 ? (len + kSplitTokens - 1) / kSplitTokens : 1;
+    if (sp < ns) process(r, h, sp, len, kSplitTokens, ns, entry, 0, pre);
     return;
   }
   auto run_item = [&](const int r, const int h, const int sp, const int len, const int split_len, const int ns) {
@@ -1327,12 +1319,14 @@ __device__ __forceinline__ void split_pass(DecodeArgs a, const int block, const 
   }
 }
 
-// Four waves to an item (quarters<T, D, G> only), for launches that leave most of
-// the chip idle.
+// Eight waves to a whole (row, kv head) (quarters<T, D, G> only), for launches of
+// few rows of two to four splits.
 template <typename T, int D, int G, int P, int TILE, bool APPEND>
 __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(2))) void paged_decode_row_kernel(DecodeArgs a) {
   split_pass<T, D, G, P, TILE, true, false, APPEND, false, false, true>(a, blockIdx.x, gridDim.x);
 }
+// Four waves to an item (quarters<T, D, G> only), for launches that leave most of
+// the chip idle.
 template <typename T, int D, int G, int P, int TILE, bool APPEND, bool ONE_SPLIT>
 __global__ __launch_bounds__(256) void paged_decode_quad_kernel(DecodeArgs a) {
   split_pass<T, D, G, P, TILE, true, false, APPEND, ONE_SPLIT, true>(a, blockIdx.x, gridDim.x);

@@ -252,9 +252,11 @@ __device__ __forceinline__ bool find_work(const PrefillArgs& a, void* lds, Work&
   const int xcd = static_cast<int>(blockIdx.x) % kXcds;
   const int pos = static_cast<int>(blockIdx.x) / kXcds;
   int before = 0;
-  if (ns <= kWaveSeqs) {
+  if (MERGE || ns <= kWaveSeqs) {
     // One sequence per lane, every wave on its own: a memory round trip and
-    // kWaveSeqs steps in registers, no barrier.
+    // kWaveSeqs steps in registers, no barrier.  A cut launch has no more
+    // sequences: at most kCus / 2 items of at least kXcds heads.
+    static_assert(kCus / 2 / kXcds <= kWaveSeqs, "a cut launch's sequences fit");
     const int s = min(lane, ns - 1);
     int r0, nq;
     seq_rows(a, s, r0, nq);
@@ -280,20 +282,19 @@ __device__ __forceinline__ bool find_work(const PrefillArgs& a, void* lds, Work&
     w.nq = __builtin_amdgcn_readlane(nq, w.seq);
     w.len = __builtin_amdgcn_readlane(len, w.seq);
     w.n = __builtin_amdgcn_readlane(n, w.seq);
-  } else {
+  } else if constexpr (!MERGE) {
     // One sequence per thread, costs and units exchanged through LDS.
     uint32_t* s_key = static_cast<uint32_t*>(lds);             // [kRankSeqs] cost, then index
     int* s_units = reinterpret_cast<int*>(s_key + kRankSeqs);  // [kRankSeqs]
     int* s_hit = s_units + kRankSeqs;                          // the workgroup's sequence: index, before
-    int r0, nq = 0, len = 0, n = 1, units = 0;
+    int r0, nq = 0, len = 0, units = 0;
     uint32_t key = 0;
     if (tid < ns) {
       seq_rows(a, tid, r0, nq);
       len = static_cast<int>(min<int64_t>(a.lens[tid], max_len));
-      n = seq_segments(len, a.max_seg);
-      units = seq_units<MERGE>(nq, n);
+      units = seq_units<MERGE>(nq, 1);
       // 23 bits of cost: longer contexts (over 2^29 keys) rank by index.
-      const uint32_t cost = static_cast<uint32_t>(segment_tiles(len, n));
+      const uint32_t cost = static_cast<uint32_t>(key_tiles(len));
       key = min(cost, (1u << 23) - 1) * kRankSeqs + (kRankSeqs - 1 - tid);
     }
     s_key[tid] = key;  // slots past ns count nothing
@@ -325,7 +326,7 @@ __device__ __forceinline__ bool find_work(const PrefillArgs& a, void* lds, Work&
     seq_rows(a, w.seq, r0, nq);
     w.row0 = uniform(r0), w.nq = uniform(nq);
     w.len = uniform(static_cast<int>(min<int64_t>(a.lens[w.seq], max_len)));
-    w.n = seq_segments(w.len, a.max_seg);
+    w.n = 1;
     __syncthreads();  // the ranking arrays are dead before the caller reuses them
   }
   const int units = seq_units<MERGE>(w.nq, w.n);
