@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 ONE_SPLIT = [0, 1, 16, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129, 161, 191, 192, 193, 224, 255, 256]
 LONGER = ONE_SPLIT + [257, 288, 320, 321, 447, 511, 512, 513, 705, 1000]
-# Past 64 splits of 256 tokens a split, and with it a quarter, doubles.
+# Past 64 splits of 256 tokens a split doubles.  Rows of more than four splits have
+# no quarters: one wave an item in every launch.
 LONG = [16384, 16385, 16640, 17000]
 
 

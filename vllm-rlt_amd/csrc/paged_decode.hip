@@ -188,8 +188,10 @@ struct DecodeArgs {
   // the layer slices.  The split pass reads a row's own new token from
   // k_new / v_new (its last token, when the write slot is the row's last
   // token slot) and the merge kernel stores it into the pages after every
-  // split has read them (in a single-split launch the row's one item stores
-  // it after its own reads), so no slot is written before it is read.
+  // split has read them.  Without a merge kernel the row's one item (one-split
+  // launches) or one workgroup (whole-row launches) stores it after the row's own
+  // reads.  So no slot is written before it is read, as long as no row reads a slot
+  // another row writes.
   const void* k_new;
   const void* v_new;
   int64_t kn_row, kn_head, kn_dim, vn_row, vn_head, vn_dim;
