@@ -248,6 +248,8 @@ def test_fp32_matrix_kernel_where_it_is_taken(hq, hkv, prefixes, chunks):
         (16, [1292], [700], True),  # 32 tiles, halves: six query tiles of 16 heads
         (16, [1284], [700], False),  # 31
         (32, [0, 700, 1300], [300, 300, 300], False),  # nine query tiles of 32 heads: 256 items without a cut
+        (16, [1600, 1600, 1600], [300, 300, 300], False),  # nine of 16 heads: halves would be 288 items
+        (16, [170, 512, 853, 1194, 1536, 1877], [143, 304, 89, 196, 35, 250], True),  # 11, of which 5 are cut: 256
     ],
 )
 def test_keys_are_cut_where_the_merge_pays(hq, prefixes, chunks, cut):

@@ -150,7 +150,8 @@ struct PrefillArgs {
   // (max in log2 units, sum) part_ml[P * total_q + i].
   f32x4* part_acc;
   float2* part_ml;
-  int max_seg;    // segments of a sequence long enough for them
+  int max_seg;    // segments of a sequence long enough for them, if that fits the CUs
+  int safe_seg;   // segments that fit them whatever the sequences are
   int cut_tiles;  // key tiles of the longest sequence from which the launch is cut
 };
 
@@ -164,8 +165,8 @@ __device__ __forceinline__ void seq_rows(const PrefillArgs& a, int s, int& row0,
 // Key segments.  A launch of few query tiles over long contexts is few work
 // items, each a long serial walk, on a chip that is mostly idle: their keys
 // are then cut into segments, every one a work item, and a merge kernel
-// combines the partials.  The host allows max_seg segments, as many as bring
-// the launch to one item per CU; a sequence takes them as long as a segment
+// combines the partials.  A launch allows max_seg segments, as many as bring
+// it to one item per CU; a sequence takes them as long as a segment
 // keeps kSegTiles key tiles (4 iterations of two, ~6 us, against the ~10 us
 // that an item spends outside its loop) and its keys are worth a merge
 // (cut_tiles).  One 512-token chunk over 16000 keys: 194 -> 82 us in 4
@@ -219,7 +220,7 @@ __device__ __forceinline__ int segment_tiles(int len, int n) {
 // items exit, and no sequence is cut.
 constexpr int kXcds = 8;
 constexpr int kRankSeqs = 512;  // ranked mode: at most this many sequences (one per thread)
-constexpr int kWaveSeqs = 16;   // ranked by every wave in registers up to here, through LDS above
+constexpr int kWaveSeqs = 16;   // (a DPP row) ranked by every wave in registers up to here, through LDS above
 constexpr int kTablePages = 4096;  // page ids staged in LDS per workgroup (65536 keys)
 constexpr int kMergeRows = 32;     // rows of a segment-merge workgroup
 
@@ -262,9 +263,19 @@ __device__ __forceinline__ bool find_work(const PrefillArgs& a, void* lds, Work&
     seq_rows(a, s, r0, nq);
     const int len = static_cast<int>(min<int64_t>(a.lens[s], max_len));
     // A launch is cut when its longest sequence is worth it, since it waits for
-    // the merge of any of them.
-    const bool cut = a.max_seg > 1 && __builtin_amdgcn_ballot_w64(key_tiles(len) >= a.cut_tiles) != 0;
-    const int n = seq_segments(len, cut ? a.max_seg : 1);
+    // the merge of any of them, and into no more items than there are CUs:
+    // three chunks of 300 rows over 1200 keys took 31.2 us uncut and 43.2 in 288
+    // halves, six ragged ones 37.4 and 32.8 in 256 (four of them cut).
+    int most = 1;
+    if (a.max_seg > 1 && __builtin_amdgcn_ballot_w64(key_tiles(len) >= a.cut_tiles) != 0) {
+      int items = lane < ns ? hpx * seq_units<false>(nq, seq_segments(len, a.max_seg)) : 0;
+      items += __builtin_amdgcn_update_dpp(0, items, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8:
+      items += __builtin_amdgcn_update_dpp(0, items, 0x112, 0xf, 0xf, true);  // lane 15 sums the
+      items += __builtin_amdgcn_update_dpp(0, items, 0x114, 0xf, 0xf, true);  // kWaveSeqs lanes
+      items += __builtin_amdgcn_update_dpp(0, items, 0x118, 0xf, 0xf, true);
+      most = __builtin_amdgcn_readlane(items, kWaveSeqs - 1) <= kCus / kXcds ? a.max_seg : a.safe_seg;
+    }
+    const int n = seq_segments(len, most);
     const int units = seq_units<MERGE>(nq, n);
     const uint32_t key = static_cast<uint32_t>(segment_tiles(len, n)) * kWaveSeqs + (kWaveSeqs - 1 - s);
     // Lanes past ns hold copies of the last sequence: q >= ns counts nothing.
@@ -1241,13 +1252,16 @@ int paged_prefill(const void* q, const int64_t* q_strides, const void* key_cache
     // a workgroup's query rows within 32-bit offsets).
     const bool dma = head_dim == 128 && max_table_width <= kTablePages && q_strides[0] >= 0 &&
                      q_strides[0] * esize * kBM < (int64_t(1) << 31);
-    // Key segments, when the caller gave room for their partials.  Sequences
-    // are expected to be no longer than max_seqlen_q says.
-    const int64_t pairs = std::max(fewest_tiles(total_q, num_seqs),
-                                   max_qt > 0 ? std::min(pairs_bound, num_seqs * max_qt) : pairs_bound);
-    const int room = split && dma && p.ranked ? segments_room(pairs, num_seqs, max_table_width, num_q_heads) : 1;
+    // Key segments, when the caller gave room for their partials: for the fewest
+    // query tiles that the rows can be, and for the most (sequences are expected to
+    // be no longer than max_seqlen_q says).
+    const int64_t most = max_qt > 0 ? std::min(pairs_bound, num_seqs * max_qt) : pairs_bound;
+    const int64_t fewest = fewest_tiles(total_q, num_seqs);
+    const int room = split && dma && p.ranked ? segments_room(fewest, num_seqs, max_table_width, num_q_heads) : 1;
     const bool may_cut = (max_table_width * kPage + kBN - 1) / kBN >= cut_tiles(room);
-    p.max_seg = may_cut ? std::min(room, segments_of(max_table_width)) : 1;
+    const int by_keys = segments_of(max_table_width);
+    p.max_seg = may_cut ? std::min(room, by_keys) : 1;
+    p.safe_seg = std::min(p.max_seg, segments_room(std::max(fewest, most), num_seqs, max_table_width, num_q_heads));
     // The table does not say how long the sequences are: once the merge has to
     // be launched, less keys are worth a cut (100 rows over 1000 keys 25.1 / 21.5 us).
     p.cut_tiles = cut_tiles(room) - 4;
