@@ -169,7 +169,7 @@ __device__ __forceinline__ void seq_rows(const PrefillArgs& a, int s, int& row0,
 // it to one item per CU; a sequence takes them as long as a segment
 // keeps kSegTiles key tiles (4 iterations of two, ~6 us, against the ~10 us
 // that an item spends outside its loop) and its keys are worth a merge
-// (cut_tiles).  One 512-token chunk over 16000 keys: 194 -> 82 us in 4
+// (cut_tiles).  One 512-token chunk over 16000 keys: 193 -> 83 us in 4
 // segments; 100 tokens over 8192 keys 123 -> 31 us in 16.  With 256 items
 // already there nothing is cut: four 512-token chunks over 8192 keys took 158 us
 // uncut and 180 us in halves, the chip being at its power limit either way.

@@ -7,10 +7,11 @@
 // and CU, so a wave spends 8192 cycles on a tile's 128 instructions, beside
 // which loading the tile straight into operand registers costs nothing that
 // LDS staging would save (K: 16 bytes of 32 rows per load; V: whole rows).
-// Three chunks of 84-176 rows over contexts of 116-583 more: 36 us, where the
+// Three chunks of 84-176 rows over contexts of 116-583 more: 37 us, where the
 // per-token path (every row a decode of its whole context) took 182 us.
 // With few rows the chip is filled from the key side, which is why a row tile
-// is 32 rows and the waves split its keys.
+// is 32 rows and the waves split its keys; with too few it is not taken at all
+// (f32_kernel_pays in paged_prefill.hip).
 //
 // Operand layouts (lane l: i = l % 32, half = l / 32).  The products sum over
 // dims, resp. keys, in any order, so the order is the one the loads come in:
