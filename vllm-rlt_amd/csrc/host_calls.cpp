@@ -166,6 +166,28 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// Workspace bytes of a prefill; rows off 16 bytes take the per-token path, whose
+// workspace is the fp32 one's.
+int64_t prefill_need(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& tables,
+                     const at::Tensor& out) {
+  const bool rows16 = aligned_rows(q) && aligned_rows(out) && aligned_rows(k) && aligned_rows(v);
+  return g_prefill_bytes(q.size(0), tables.size(0), tables.size(1), q.size(1), k.size(2), q.size(2), k.size(1),
+                         rows16 ? code_of(q.scalar_type()) : int{RLT_FLOAT32});
+}
+
+// prefill_bytes(q, key, value, tables): what prefill() needs of a given workspace.
+PyObject* prefill_bytes(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 4 || modes_active()) Py_RETURN_NONE;
+  const at::Tensor* in[4];
+  for (int i = 0; i < 4; ++i)
+    if (!(in[i] = plain(args[i]))) Py_RETURN_NONE;
+  const at::Tensor &q = *in[0], &k = *in[1], &v = *in[2], &tables = *in[3];
+  if (q.dim() != 3 || k.dim() != 4 || v.dim() != 4 || tables.dim() != 2 || code_of(q.scalar_type()) < 0) Py_RETURN_NONE;
+  return PyLong_FromLongLong(prefill_need(q, k, v, tables, q));
+  END_HANDLE_TH_ERRORS
+}
+
 // prefill(q, key, value, tables, lengths, cu, max_seqlen_q, out, scale, stream,
 //         workspace): the workspace for key segments or the per-token path is the
 // given one when it is large enough, allocated here for None.
@@ -189,10 +211,7 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   at::Tensor out;
   if (!result_like(args[7], q, &out)) Py_RETURN_NONE;
   const int code = code_of(q.scalar_type());
-  // Rows off 16 bytes take the per-token path, whose workspace is the fp32 one's.
-  const bool rows16 = aligned_rows(q) && aligned_rows(out) && aligned_rows(k) && aligned_rows(v);
-  const int sized = rows16 ? code : int{RLT_FLOAT32};
-  const int64_t need = g_prefill_bytes(total, nseq, tables.size(1), hq, hkv, d, k.size(1), sized);
+  const int64_t need = prefill_need(q, k, v, tables, out);
   at::Tensor workspace;
   if (args[10] != Py_None) {
     const at::Tensor* w = plain(args[10]);
@@ -285,6 +304,7 @@ PyMethodDef kMethods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
     {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(decode)), METH_FASTCALL, nullptr},
     {"prefill", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(prefill)), METH_FASTCALL, nullptr},
+    {"prefill_bytes", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(prefill_bytes)), METH_FASTCALL, nullptr},
     {"rope", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(rope)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -180,15 +180,20 @@ class HipPagedAttention:
                 workspace=self.reserve(need) if need else None, batch_invariant=True,
             )
         # Under capture the steps below note that a graph reads the workspace.
-        if self._workspace is not None and q.is_cuda and not torch._C._cuda_isCurrentStreamCapturing():
+        if q.is_cuda and not torch._C._cuda_isCurrentStreamCapturing():
             host, stream = ops._host_calls(q)
-            if host is not None:
-                out = host.prefill(
-                    q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None,
-                    stream, self._workspace,
-                )
-                if out is not None:
-                    return ops._finish(out, "rlt_paged_prefill")
+            args = (q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None, stream)
+            out = None
+            if host is not None and self._workspace is not None:
+                out = host.prefill(*args, self._workspace)
+            if host is not None and out is None:
+                need = host.prefill_bytes(q, key_cache, value_cache, block_tables)
+                if need:  # a first call, or one that outgrows the workspace
+                    out = host.prefill(*args, self.reserve(need))
+                elif need == 0 and self._workspace is None:
+                    out = host.prefill(*args, None)
+            if out is not None:
+                return ops._finish(out, "rlt_paged_prefill")
         need = ops.prefill_split_workspace_bytes(*self._prefill_shape(q, key_cache, value_cache, block_tables))
         return ops._paged_prefill(
             q, key_cache, value_cache, block_tables, context_lengths, cu_seqlens_q, max_seqlen_q, None, None,
