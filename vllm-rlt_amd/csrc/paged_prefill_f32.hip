@@ -7,7 +7,7 @@
 // and CU, so a wave spends 8192 cycles on a tile's 128 instructions, beside
 // which loading the tile straight into operand registers costs nothing that
 // LDS staging would save (K: 16 bytes of 32 rows per load; V: whole rows).
-// Three chunks of 84-176 rows over contexts of 116-583 more: 37 us, where the
+// Three chunks of 84-176 rows over contexts of 116-583 more: 36 us, where the
 // per-token path (every row a decode of its whole context) took 182 us.
 // With few rows the chip is filled from the key side, which is why a row tile
 // is 32 rows and the waves split its keys; with too few it is not taken at all
@@ -153,19 +153,22 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
 
   // Tiles with keys that some row does not see.  P = 0 keeps a masked key's V
   // out of a row only while it is finite, so what is not leaves the products
-  // here, and the store adds it to the rows that see it.
+  // here, and the store adds it to the rows that see it.  One product an element
+  // finds out whether there is any (comparing each cost 2% of the kernel).
   auto confine = [&](int n) __attribute__((always_inline)) {
     if (kKeys * (wave + kWaves * n) + kKeys - 1 <= open) return;
-    bool odd = false;
+    float t = 0.f;  // 0 times what is not finite is a NaN
 #pragma unroll
     for (int u = 0; u < 8; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool finite = (__float_as_uint(vr[u][e]) & 0x7f800000u) != 0x7f800000u;
-        odd |= !finite;
-        vr[u][e] = finite ? vr[u][e] : 0.f;
-      }
-    if (odd) lds_odd = 1;
+      for (int e = 0; e < 4; ++e) t = fmaf(vr[u][e], 0.f, t);
+    if (__builtin_amdgcn_ballot_w64(t != t) == 0) return;
+    lds_odd = 1;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if ((__float_as_uint(vr[u][e]) & 0x7f800000u) == 0x7f800000u) vr[u][e] = 0.f;
   };
 
   const int mine = ntiles > wave ? (ntiles - wave + kWaves - 1) / kWaves : 0;
